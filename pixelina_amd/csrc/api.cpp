@@ -1356,13 +1356,16 @@ int attention_run(pixhip_session* s, const float* q, size_t rows, const float* k
         release();
         return rc;
     }
-    if ((rc = grow(s,&s->attn,&s->attn_bytes,pixhip::attention_workspace_bytes(rows,keys,heads,kv_heads,dim)))) {
+    const void* seen = nullptr;
+    const bool resident = device_visible(s,kd,&seen) && device_visible(s,vd,&seen);
+    if ((rc = grow(s,&s->attn,&s->attn_bytes,
+                   pixhip::attention_workspace_bytes(keys,heads,kv_heads,dim,ranges,count,resident)))) {
         release();
         return rc;
     }
     hipError_t e = pixhip::launch_attention(static_cast<const float*>(qd),static_cast<const float*>(kd),static_cast<const float*>(vd),
-                                            static_cast<float*>(out),rows,keys,heads,kv_heads,dim,ranges,count,query_offset,s->attn,
-                                            s->stream);
+                                            static_cast<float*>(out),rows,keys,heads,kv_heads,dim,ranges,count,query_offset,resident,
+                                            s->attn,s->stream);
     release();
     if (e == hipErrorInvalidValue) return fail(PIXHIP_ERR_ARGUMENT,"attention shape beyond the kernel's 32-bit index range");
     PIX_HIP(e,"attention");

@@ -250,13 +250,16 @@ struct AttnRange {
 };
 // Head size rounded up to the kernel's (64 or 128); 0 when not supported.
 int attention_dim_pad(size_t dim);
-// Workspace of launch_attention (bf16 split planes of Q, K and V^T).
-size_t attention_workspace_bytes(size_t rows, size_t keys, size_t heads, size_t kv_heads, size_t dim);
+// Workspace of launch_attention (bf16 split planes of K and V^T where a range
+// needs them, key pieces' partial results).
+size_t attention_workspace_bytes(size_t keys, size_t heads, size_t kv_heads, size_t dim, const AttnRange* ranges, size_t count,
+                                 bool resident);
 // out [rows][heads*dim] for q [rows][heads*dim], k and v [keys][kv_heads*dim]
 // (device pointers), one kernel launch per range (a range's rows only).
+// `resident`: k and v are device memory (not pinned host memory).
 hipError_t launch_attention(const float* q, const float* k, const float* v, float* out, size_t rows, size_t keys, size_t heads,
-                            size_t kv_heads, size_t dim, const AttnRange* ranges, size_t count, size_t query_offset, void* workspace,
-                            hipStream_t s);
+                            size_t kv_heads, size_t dim, const AttnRange* ranges, size_t count, size_t query_offset, bool resident,
+                            void* workspace, hipStream_t s);
 
 // matvec.hip
 hipError_t launch_matvec_q5_K(const PlanarQ5K& w, const float* x, size_t N, size_t K, const Output& out, hipStream_t s);

@@ -120,6 +120,49 @@ def test_wide_head_ranges(sess):
     assert err <= TOL
 
 
+@pytest.mark.parametrize("rows,keys,heads,kvh,dim,causal,offset", [
+    (1, 1, 4, 4, 64, True, 0),         # one key
+    (1, 15, 3, 1, 128, False, 0),      # three queries in a group of four, keys below one batch
+    (1, 65, 16, 2, 72, True, 64),      # eight queries, head size 72, one key past a whole step
+    (1, 2501, 32, 8, 128, True, 2500),  # a decode step: many key pieces
+    (2, 1024, 2, 1, 4, True, 1022),    # the smallest head size of the few-query kernel
+    (3, 200, 6, 2, 40, True, 197),     # nine queries: two groups, causal rows with different limits
+    (4, 130, 8, 1, 128, False, 0),     # 32 queries: the kernel's most
+    (33, 130, 1, 1, 128, True, 97),    # 33 queries: the tiled kernel
+    (5, 300, 14, 2, 80, True, 295),    # 35 packed queries, heads of 80 sharing a tile
+    (128, 700, 28, 4, 128, True, 572),  # a prefill chunk, seven heads per kv head in one query list
+    (70, 70, 6, 2, 64, True, 0),       # packed, ragged, head size 64
+])
+def test_short_ranges_against_oracle(sess, rows, keys, heads, kvh, dim, causal, offset):
+    """Decode steps and short chunks behind a cache: the few-query kernel (rows x
+    grouped heads up to 32, fp32 products) and the tiled kernel's packed heads."""
+    rng = np.random.default_rng(rows * 31 + keys)
+    q, k, v = qkv(rng, rows, keys, heads, kvh, dim)
+    ranges = [(0, rows, keys, int(causal))]
+    print(f"rows={rows} keys={keys} heads={heads}/{kvh} dim={dim} causal={causal} offset={offset}", flush=True)
+    y = gpu_attention(sess, q, k, v, heads, kvh, ranges=ranges, query_offset=offset)
+    ref = attention(oracle(), "orc", q, k, v, heads, kvh, ranges, offset)
+    err = row_rel_error(y, ref).max()
+    print(f"  rel={err:.2e}", flush=True)
+    assert err <= TOL
+    y2 = gpu_attention(sess, q, k, v, heads, kvh, ranges=ranges, query_offset=offset)
+    assert np.array_equal(y.view(np.uint32), y2.view(np.uint32)), "repeats differ"
+
+
+def test_short_and_long_ranges_together(sess):
+    """Ranges of one call on different kernels: 2 rows (few queries), 90 rows
+    (tiled), 1 row limited to a key prefix."""
+    rng = np.random.default_rng(5)
+    rows, keys, heads, kvh, dim, offset = 93, 150, 4, 2, 128, 30
+    q, k, v = qkv(rng, rows, keys, heads, kvh, dim)
+    ranges = [(0, 2, 150, 1), (2, 92, 150, 1), (92, 93, 7, 0)]
+    y = gpu_attention(sess, q, k, v, heads, kvh, ranges=ranges, query_offset=offset)
+    ref = attention(oracle(), "orc", q, k, v, heads, kvh, ranges, offset)
+    err = row_rel_error(y, ref).max()
+    print(f"rel={err:.2e}", flush=True)
+    assert err <= TOL
+
+
 @pytest.mark.parametrize("tokens,dim", [(16384, 512), (4096, 384)])
 def test_vae_mid_block_sampled(sess, tokens, dim):
     """The VAE mid-block attention: one head of 512 channels over the 128 x 128
