@@ -19,6 +19,7 @@ SOURCES = [
     "csrc/repack.hip",
     "csrc/gemm.hip",
     "csrc/gemm_kq.hip",
+    "csrc/gemm_kq_rows.hip",
     "csrc/matvec.hip",
     "csrc/fuse.hip",
     "csrc/ops.hip",
@@ -70,11 +71,13 @@ def _compile(src):
 # build fails if the compiler spills any (the integer-sum debug variants drain
 # the counter completely and are exempt).  The attention kernels drain it
 # completely too, but sit at the register limit, where a spill would mean
-# scratch traffic in the key loop; they are checked as well.
+# scratch traffic in the key loop; they are checked as well, as are the few-token
+# kernels (a tile that spilled ran three times slower).
 NO_SPILL = {
     "csrc/attention.hip": ("attn_kernelILi128ELi1E", "attn_kernelILi128ELi2E", "attn_kernelILi64ELi1E", "attn_kernelILi64ELi2E", "attn_wide_kernelILi128E", "attn_wide_kernelILi96E",
                            "attn_wide_kernelILi64E"),
     "csrc/gemm_kq.hip": ("gemm_kq_kernelILb1ELb0E", "gemm_kq_kernelILb0ELb0E"),
+    "csrc/gemm_kq_rows.hip": ("gemm_kq_rows_kernel",),
     "csrc/gemm.hip": ("gemm_kernelILb0E", "gemm_small_kernel"),
 }
 

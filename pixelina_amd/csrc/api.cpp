@@ -579,7 +579,8 @@ int multiply_stage(pixhip_session* s, pixhip_weight* w, size_t columns, const pi
         return fail(PIXHIP_ERR_STATE,"no quantized activations of this shape: run the QUANTIZE stage first");
     int rc = ensure_gemm_form(s,w);
     if (rc) return rc;
-    const size_t part_bytes = kind == 2 && pixhip::gemm_q8_0_grouped(columns,w->rows)
+    const bool few = kind == 1 && pixhip::gemm_kq_rows(columns,w->rows,w->inner);
+    const size_t part_bytes = few || (kind == 2 && pixhip::gemm_q8_0_grouped(columns,w->rows))
                                   ? 0
                                   : pixhip::gemm_split_bytes(columns,w->rows,round_up(w->inner,64));
     if (part_bytes) {
@@ -588,7 +589,9 @@ int multiply_stage(pixhip_session* s, pixhip_weight* w, size_t columns, const pi
     }
     float* part = part_bytes? static_cast<float*>(s->partial) : nullptr;
     hipError_t e;
-    if (w->type == PIX_Q5_K) e = pixhip::launch_gemm_q5_K(s->a8k,w->q5,columns,w->rows,w->inner,out,part,s->stream);
+    if (few && w->type == PIX_Q5_K) e = pixhip::launch_gemm_rows_q5_K(s->a8k,w->q5,columns,w->rows,w->inner,out,s->stream);
+    else if (few) e = pixhip::launch_gemm_rows_q6_K(s->a8k,w->q6,columns,w->rows,w->inner,out,s->stream);
+    else if (w->type == PIX_Q5_K) e = pixhip::launch_gemm_q5_K(s->a8k,w->q5,columns,w->rows,w->inner,out,part,s->stream);
     else if (w->type == PIX_Q6_K) e = pixhip::launch_gemm_q6_K(s->a8k,w->q6,columns,w->rows,w->inner,out,part,s->stream);
     else e = pixhip::launch_gemm_q8_0(s->a80,w->q80,columns,w->rows,w->inner,out,part,s->stream);
     PIX_HIP(e,"GEMM launch");
@@ -630,7 +633,9 @@ int matvec(pixhip_session* s, pixhip_weight* w, const float* x, const pixhip::Ou
 // activations are a view of the session's buffers for all rows (which they
 // hold afterwards, as after an unchunked call) and its GEMM reads that view.
 // Taken only when the chunks' GEMMs and the whole one run the same kernel
-// form with no split-K, so every output is the same bits either way.
+// form with no split-K, so every output is the same bits either way.  (Grids
+// small enough for the few-token K-quant form split, or have one super-block,
+// which that form adds the same way.)
 size_t pipe_chunk(size_t columns) { return round_up((columns + kPipeChunks - 1) / kPipeChunks,kTileM); }
 
 bool pipeline_ok(const pixhip_weight* w, size_t columns)
@@ -1148,8 +1153,12 @@ int pixhip_matmul_ex_noalloc(pixhip_session* s, const pixhip_weight* wc, const f
         const pixhip::Act8K a = {reinterpret_cast<int8_t*>(base + qs),reinterpret_cast<float*>(base + d),
                                  reinterpret_cast<_Float16*>(base + bs),mpad};
         PIX_HIP(pixhip::launch_quantize_q8_K(x,columns,K,a,nullptr,s->stream),"quantize Q8_K");
-        e = w->type == PIX_Q5_K? pixhip::launch_gemm_q5_K(a,w->q5,columns,w->rows,K,out,nullptr,s->stream)
-                               : pixhip::launch_gemm_q6_K(a,w->q6,columns,w->rows,K,out,nullptr,s->stream);
+        if (pixhip::gemm_kq_rows(columns,w->rows,K))
+            e = w->type == PIX_Q5_K? pixhip::launch_gemm_rows_q5_K(a,w->q5,columns,w->rows,K,out,s->stream)
+                                   : pixhip::launch_gemm_rows_q6_K(a,w->q6,columns,w->rows,K,out,s->stream);
+        else
+            e = w->type == PIX_Q5_K? pixhip::launch_gemm_q5_K(a,w->q5,columns,w->rows,K,out,nullptr,s->stream)
+                                   : pixhip::launch_gemm_q6_K(a,w->q6,columns,w->rows,K,out,nullptr,s->stream);
     }
     PIX_HIP(e,"GEMM launch");
     PIX_HIP(hipEventRecord(g_scratch_event[dev],s->stream),"hipEventRecord (scratch order)");

@@ -771,7 +771,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs g)
     }
 }
 
-static int device_cus()
+int device_cus()
 {
     static int cus = 0;
     if (!cus) {

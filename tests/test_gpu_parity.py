@@ -189,3 +189,28 @@ def test_copy_device_is_exact(sess):
         assert np.array_equal(dst.download(np.uint8, nbytes), data)
         src.free()
         dst.free()
+
+
+@pytest.mark.parametrize("wtype", [Q5_K, Q6_K])
+@pytest.mark.parametrize("m,n,k", [
+    (2, 7, 256),        # one super-block, fewer features than a tile
+    (3, 97, 1536),      # more super-blocks than waves, a ragged feature tile
+    (16, 12300, 512),   # three feature tiles a workgroup, the last of them past the padding
+    (17, 8200, 768),    # two token tiles, two feature tiles
+    (37, 4096, 1280),   # three token tiles
+    (48, 9000, 256),
+    (96, 130, 1024),    # six token tiles
+    (100, 4000, 512),
+    (128, 640, 2048),   # eight token tiles
+    (128, 12288, 256),  # four token and two feature tiles
+    (250, 33, 1024),    # several tiles of tokens, up to the padded rows
+    (700, 64, 512),
+])
+def test_few_token_kquant(sess, wtype, m, n, k):
+    # exact integer sums, fp32 sums over k / 256 <= 8 super-blocks in another order than the oracle's:
+    # 8 * 2^-24 relative to the terms, which exceed a row's largest output by less than 10
+    rng = np.random.default_rng(m * 31 + n)
+    wb = pack(wtype, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    ref = quant_matmul(oracle(), "orc", wb, wtype, x, n)
+    assert row_rel_error(gpu_matmul(sess, wb, wtype, x, n), ref).max() <= 5e-6
