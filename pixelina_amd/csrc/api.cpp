@@ -131,7 +131,7 @@ struct pixhip_weight {
     size_t resident = 0;
     uint64_t used = 0;
     // convolution weights (F32 / F16 / BF16, [cout][cin * ky * kx]): the
-    // split-bf16 planes the implicit GEMM reads, built on first use
+    // 16-bit planes the implicit GEMM reads, built on first use
     bool conv = false;
     uint32_t kernel_x = 0, kernel_y = 0, cin = 0;
     void* conv_planes = nullptr;
@@ -1852,17 +1852,18 @@ int pixhip_shortcut(pixhip_session* s, const float* source, size_t width, size_t
 
 namespace {
 
-// The split-bf16 planes of a convolution weight, built from its file bytes.
+// The 16-bit planes of a convolution weight, built from its file bytes.
 int ensure_conv_form(pixhip_session* s, pixhip_weight* w)
 {
     if (w->conv_planes) return PIXHIP_OK;
     int rc = ensure_raw(s,w);
     if (rc) return rc;
     const size_t plane = w->conv_npad * w->conv_kp * sizeof(uint16_t);
-    if ((rc = weight_alloc(s,w,2 * plane,&w->conv_planes))) return rc;
+    const int kind = pixhip::conv_weight_kind(w->type,(int)w->cin);
+    if ((rc = weight_alloc(s,w,(kind == pixhip::kConvSplit? 2 : 1) * plane,&w->conv_planes))) return rc;
     uint16_t* hi = static_cast<uint16_t*>(w->conv_planes);
     PIX_HIP(pixhip::launch_conv_form(w->raw,w->type,(int)w->kernel_x,(int)w->kernel_y,(int)w->cin,(int)w->rows,(int)w->conv_kp,
-                                     (int)w->conv_npad,hi,hi + plane / sizeof(uint16_t),s->stream),
+                                     (int)w->conv_npad,kind,hi,hi + plane / sizeof(uint16_t),s->stream),
             "convolution weight form");
     return release_raw(s,w);
 }
@@ -1970,7 +1971,8 @@ int pixhip_conv2d(pixhip_session* s, const pixhip_weight* wc, const float* input
     pixhip::ConvArgs a{};
     a.x = static_cast<const float*>(in);
     a.wh = static_cast<const uint16_t*>(w->conv_planes);
-    a.wl = a.wh + w->conv_npad * w->conv_kp;
+    a.kind = pixhip::conv_weight_kind(w->type,(int)w->cin);
+    a.wl = a.kind == pixhip::kConvSplit? a.wh + w->conv_npad * w->conv_kp : nullptr;
     a.bias = static_cast<const float*>(b);
     a.y = static_cast<float*>(out);
     a.W = (int)width;

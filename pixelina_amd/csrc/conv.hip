@@ -10,11 +10,15 @@
 // image into LDS, with the inner dimension ordered (ky, kx, c) so that a stage
 // of 32 is one kernel tap over 32 consecutive channels (one 128-byte run per
 // pixel) whenever channels % 32 == 0 -- the weight is stored in that order
-// when it is made resident.  Products run as attention's do: every fp32
-// operand split into bf16 halves (hi = bf16(x), lo = bf16(x - hi)) and
-// a*b = hi*hi + hi*lo + lo*hi on v_mfma_f32_32x32x16_bf16 with fp32
-// accumulation, about 2^-16 relative per product (the weight halves are made
-// once, at upload; F16 and BF16 weights are exact in them).
+// when it is made resident.  fp32 operands are split into bf16 halves (hi =
+// bf16(x), lo = bf16(x - hi)) and a*b = hi*hi + hi*lo + lo*hi on
+// v_mfma_f32_32x32x16_bf16 with fp32 accumulation, about 2^-16 relative per
+// product.  The matrix core bounds the large layers, so weights that have fewer
+// bits than an fp32 take fewer products: BF16 weights are one bf16 plane (two
+// products, the same sums), F16 weights one fp16 plane that multiplies an image
+// split in fp16 under a scale (two products; conv_body_ring).  256^2 pixels,
+// 512 -> 512, 3x3: three products 889 us, two fp16 721 (error against 64 bits
+// 3.8e-6 -> 6.2e-7), two bf16 678.
 //
 // Tile: 128 pixels x 128 output channels x 32 inner per stage, 4 waves of
 // 64 x 64 (2 x 2 MFMA tiles).  The image kernel (images below 2 GiB) keeps one
@@ -120,6 +124,26 @@ __device__ __forceinline__ void halves2(float a, float b, uint32_t& hi, uint32_t
     lo = pack_bf16(a - __uint_as_float(hi << 16),b - __uint_as_float(hi & 0xFFFF0000u));
 }
 
+// Eight fp16 values as bf16 halves (exact: 11 bits are 8 and 3).
+__device__ __forceinline__ void half_planes(cu32x4 v, cu32x4& hi, cu32x4& lo)
+{
+    const v8h h = __builtin_bit_cast(v8h,v);
+    uint32_t a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) halves2((float)h[2 * q],(float)h[2 * q + 1],a[q],b[q]);
+    hi = cu32x4{a[0],a[1],a[2],a[3]};
+    lo = cu32x4{b[0],b[1],b[2],b[3]};
+}
+
+// The fp16 split of a pair: hi truncated to fp16, lo = the remainders truncated
+// to fp16: 2^-20 of the value, or fp16's last place 2^-24 where that is more.
+__device__ __forceinline__ void halves2_f16(float a, float b, uint32_t& hi, uint32_t& lo)
+{
+    const auto h = __builtin_amdgcn_cvt_pkrtz(a,b);
+    hi = __builtin_bit_cast(uint32_t,h);
+    lo = __builtin_bit_cast(uint32_t,__builtin_amdgcn_cvt_pkrtz(a - (float)h[0],b - (float)h[1]));
+}
+
 __device__ __forceinline__ float weight_value(const uint8_t* raw, uint32_t type, size_t index)
 {
     if (type == PIX_F32) {
@@ -133,11 +157,21 @@ __device__ __forceinline__ float weight_value(const uint8_t* raw, uint32_t type,
 
 }  // namespace
 
-// Weight form: planes [npad][kp] of bf16 (hi, lo); row n, column k' = (ky *
+// The form a weight of `type` is held in: BF16 weights are one bf16 plane, F16
+// weights one fp16 plane where the image kernel reads them (whole stages of 32
+// channels), everything else the two split planes.
+int conv_weight_kind(uint32_t type, int cin)
+{
+    if (type == PIX_BF16) return kConvBf16;
+    return type == PIX_F16 && cin % kCK == 0? kConvHalf : kConvSplit;
+}
+
+// Weight form: planes [npad][kp] of bf16 (hi, lo; the fp16 or bf16 plane alone
+// where the weight has only one); row n, column k' = (ky *
 // kernel_x + kx) * cin + c holds weight[n][(c * kernel_y + ky) * kernel_x + kx]
 // of the GGUF / safetensors tensor; zero past cout and inner.
 __global__ __launch_bounds__(256) void conv_form_kernel(const uint8_t* __restrict__ raw, uint32_t type, int kx_n, int ky_n, int cin,
-                                                        int cout, int kp, int npad, uint16_t* __restrict__ hi, uint16_t* __restrict__ lo)
+                                                        int cout, int kp, int npad, int kind, uint16_t* __restrict__ hi, uint16_t* __restrict__ lo)
 {
     const size_t inner = (size_t)cin * kx_n * ky_n, total = (size_t)npad * kp, step = (size_t)gridDim.x * blockDim.x;
     for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += step) {
@@ -147,19 +181,23 @@ __global__ __launch_bounds__(256) void conv_form_kernel(const uint8_t* __restric
             const int c = k % cin, tap = k / cin, kx = tap % kx_n, ky = tap / kx_n;
             w = weight_value(raw,type,(size_t)n * inner + ((size_t)c * ky_n + ky) * kx_n + kx);
         }
+        if (kind == kConvHalf) {
+            hi[e] = float_to_half_bits(w);  // (exact: the value was fp16)
+            continue;
+        }
         uint32_t h, l;
         halves(w,h,l);
         hi[e] = (uint16_t)h;
-        lo[e] = (uint16_t)l;
+        if (kind == kConvSplit) lo[e] = (uint16_t)l;
     }
 }
 
-hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad,
+hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad, int kind,
                             uint16_t* hi, uint16_t* lo, hipStream_t s)
 {
     const size_t total = (size_t)npad * kp;
     const unsigned grid = (unsigned)std::min<size_t>((total + 255) / 256,(size_t)1 << 20);
-    conv_form_kernel<<<dim3(grid),dim3(256),0,s>>>(static_cast<const uint8_t*>(raw),type,kernel_x,kernel_y,cin,cout,kp,npad,hi,lo);
+    conv_form_kernel<<<dim3(grid),dim3(256),0,s>>>(static_cast<const uint8_t*>(raw),type,kernel_x,kernel_y,cin,cout,kp,npad,kind,hi,lo);
     return hipGetLastError();
 }
 
@@ -231,6 +269,7 @@ __device__ __forceinline__ void conv_body(const ConvArgs& a)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int q = t + 256 * (j & 1), row = q / 4, part = q % 4;
+            if (j >= 2 && a.kind != kConvSplit) continue;  // one plane
             const uint16_t* plane = (j < 2)? a.wh : a.wl;
             rb[j] = *reinterpret_cast<const cu32x4*>(plane + (size_t)(n0 + row) * a.Kp + k0 + part * 8);
         }
@@ -257,6 +296,12 @@ __device__ __forceinline__ void conv_body(const ConvArgs& a)
                 st[row * kCRow + col] = (uint16_t)h;
                 st[PA + row * kCRow + col] = (uint16_t)l;
             }
+        }
+        if (a.kind == kConvHalf) {
+#pragma unroll
+            for (int j = 0; j < 2; j++) half_planes(rb[j],rb[j],rb[j + 2]);
+        } else if (a.kind == kConvBf16) {
+            rb[2] = rb[3] = cu32x4{0,0,0,0};
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -335,19 +380,36 @@ __device__ __forceinline__ void conv_body(const ConvArgs& a)
 // stores to LDS wait on loads issued a whole stage earlier.  LDS: one A stage
 // (hi, lo: 20 KB) + two B slots (hi, lo: 16 KB each) = 52 KB, three
 // workgroups per CU.
-__device__ __forceinline__ void conv_body_ring(const ConvArgs& a)
+//
+// FORM is how the products are formed:
+//   kConvSplit  three bf16 products of split weights and image;
+//   kConvBf16   the weight is one bf16 plane: two products, the same sums;
+//   kConvHalf   the weight is one fp16 plane: two fp16 products of the image
+//               times `scale` (a power of two), split as hi + lo in fp16.
+//               Returns true, without an output, where an output pixel's
+//               inputs leave the range in which that split is at least as fine
+//               as the bf16 one: their largest |x * scale| above 2^15, or
+//               below 2^-6 and not zero (fp16's last place, 2^-24, is then
+//               more than 2^-18 of it);
+//   kConvWiden  the second try of those tiles: the plane widened to bf16
+//               halves, three bf16 products, one stage at a time.
+constexpr int kConvWiden = 3;
+template <int FORM>
+__device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, uint16_t (&lds)[2 * 128 * kCRow],
+                                               uint16_t (&bslot0)[2 * kCN * 32], uint16_t (&bslot1)[2 * kCN * 32])
 {
+    constexpr bool WIDEN = FORM == kConvWiden, SPLIT = FORM == kConvSplit || WIDEN, HALF = FORM == kConvHalf;
+    constexpr int CHUNKS = SPLIT? 4 : 2;  // weight transfers of a wave per stage
     constexpr int BM = 128, AV = 4;
     constexpr int PA = BM * kCRow;   // bf16 per A plane (80-byte rows)
     constexpr int PB = kCN * 32;     // bf16 per B plane (64-byte rows)
-    // (separate arrays: the compiler can then tell the image stores from the
-    // transfers in flight into the ring)
-    __shared__ __attribute__((aligned(1024))) uint16_t lds[2 * PA];
-    __shared__ __attribute__((aligned(1024))) uint16_t bslot0[2 * PB];  // ring slots: planes hi, lo
-    __shared__ __attribute__((aligned(1024))) uint16_t bslot1[2 * PB];
-    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), lr = lane & 31, hh = lane >> 5;
+    // (opaque: values shared with the first try would sit in registers through its loop)
+    int t = threadIdx.x;
+    uint32_t tile_m = blockIdx.x;
+    if constexpr (WIDEN) __asm__ volatile("" : "+v"(t), "+s"(tile_m));
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), lr = lane & 31, hh = lane >> 5;
     const int wm = wave & 1, wn = wave >> 1;
-    const long long m0 = (long long)blockIdx.x * BM;
+    const long long m0 = (long long)tile_m * BM;
     const int n0 = blockIdx.y * kCN;
 
     int iy0[AV], ix0[AV];
@@ -365,18 +427,18 @@ __device__ __forceinline__ void conv_body_ring(const ConvArgs& a)
     }
     const uint32_t wbytes = (uint32_t)((size_t)a.Npad * a.Kp * 2);
     const CRsrc rx = conv_rsrc(a.x,(uint32_t)((size_t)a.W * a.H * a.C * 4));
-    const CRsrc rwh = conv_rsrc(a.wh,wbytes), rwl = conv_rsrc(a.wl,wbytes);
-    // B DMA: the stage's 16 chunks of 1 KB (plane c / 8, rows 16 (c % 8) ..
-    // +15), chunk c = wave + 4i; lane l lands at row l / 4, physical piece l % 4
-    uint32_t bvo[4];
+    const CRsrc rwh = conv_rsrc(a.wh,wbytes), rwl = conv_rsrc(FORM == kConvSplit? a.wl : a.wh,wbytes);
+    // B DMA: the stage's 16 (one plane: 8) chunks of 1 KB (plane c / 8, rows
+    // 16 (c % 8) .. +15), chunk c = wave + 4i; lane l lands at row l / 4, physical piece l % 4
+    uint32_t bvo[CHUNKS];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < CHUNKS; i++) {
         const int c = wave + 4 * i, row = 16 * (c % 8) + lane / 4, logical = (lane % 4) ^ ((row >> 2) & 3);
         bvo[i] = ((uint32_t)(n0 + row) * (uint32_t)a.Kp + 8u * (uint32_t)logical) * 2u;
     }
     auto issue_b = [&](int stage, int slot) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < CHUNKS; i++) {
             const int c = wave + 4 * i;
             uint16_t* dst = (slot? bslot1 : bslot0) + (c / 8) * PB + (c % 8) * 512;
             conv_dma(c < 8? rwh : rwl,dst,bvo[i],(uint32_t)(stage * kCK * 2));
@@ -405,13 +467,24 @@ __device__ __forceinline__ void conv_body_ring(const ConvArgs& a)
             ra[i] = make_float4(__uint_as_float(v.x),__uint_as_float(v.y),__uint_as_float(v.z),__uint_as_float(v.w));
         }
     };
+    float top[HALF? AV : 1];  // largest |x * scale| of this thread's share of each pixel's inputs
+#pragma unroll
+    for (int i = 0; i < (HALF? AV : 1); i++) top[i] = 0.0f;
     auto store_a = [&](const float4 (&ra)[AV]) {
 #pragma unroll
         for (int i = 0; i < AV; i++) {
             const int row = t / 8 + 32 * i, col = (t % 8) * 4;
             uint32_t h01, l01, h23, l23;
-            halves2(ra[i].x,ra[i].y,h01,l01);
-            halves2(ra[i].z,ra[i].w,h23,l23);
+            if constexpr (HALF) {
+                const float x0 = ra[i].x * scale, x1 = ra[i].y * scale, x2 = ra[i].z * scale, x3 = ra[i].w * scale;
+                top[i] = __builtin_fmaxf(__builtin_fmaxf(top[i],__builtin_fabsf(x0)),__builtin_fabsf(x1));
+                top[i] = __builtin_fmaxf(__builtin_fmaxf(top[i],__builtin_fabsf(x2)),__builtin_fabsf(x3));
+                halves2_f16(x0,x1,h01,l01);
+                halves2_f16(x2,x3,h23,l23);
+            } else {
+                halves2(ra[i].x,ra[i].y,h01,l01);
+                halves2(ra[i].z,ra[i].w,h23,l23);
+            }
             *reinterpret_cast<uint2*>(lds + row * kCRow + col) = make_uint2(h01,h23);
             *reinterpret_cast<uint2*>(lds + PA + row * kCRow + col) = make_uint2(l01,l23);
         }
@@ -427,68 +500,114 @@ __device__ __forceinline__ void conv_body_ring(const ConvArgs& a)
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
             const int col = ks * 16 + 8 * hh;
-            cbf16x8 ah[2], al[2], bh[2], bl[2];
+            cu32x4 ah[2], al[2], bh[2], bl[2];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int row = wn * 64 + j * 32 + lr;
                 const int at = row * 32 + (((2 * ks + hh) ^ ((row >> 2) & 3)) << 3);
-                bh[j] = *reinterpret_cast<const cbf16x8*>(bs + at);
-                bl[j] = *reinterpret_cast<const cbf16x8*>(bs + PB + at);
+                bh[j] = *reinterpret_cast<const cu32x4*>(bs + at);
+                if constexpr (SPLIT) bl[j] = *reinterpret_cast<const cu32x4*>(bs + PB + at);
             }
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 const int row = wm * 64 + i * 32 + lr;
-                ah[i] = *reinterpret_cast<const cbf16x8*>(lds + row * kCRow + col);
-                al[i] = *reinterpret_cast<const cbf16x8*>(lds + PA + row * kCRow + col);
+                ah[i] = *reinterpret_cast<const cu32x4*>(lds + row * kCRow + col);
+                al[i] = *reinterpret_cast<const cu32x4*>(lds + PA + row * kCRow + col);
             }
+            auto product = [](cu32x4 x, cu32x4 w, v16f c) {
+                if constexpr (HALF) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h,x),__builtin_bit_cast(v8h,w),c,0,0,0);
+                else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(cbf16x8,x),__builtin_bit_cast(cbf16x8,w),c,0,0,0);
+            };
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i],bh[j],acc[i][j],0,0,0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i],bl[j],acc[i][j],0,0,0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i],bh[j],acc[i][j],0,0,0);
+                    acc[i][j] = product(ah[i],bh[j],acc[i][j]);
+                    if constexpr (SPLIT) acc[i][j] = product(ah[i],bl[j],acc[i][j]);
+                    acc[i][j] = product(al[i],bh[j],acc[i][j]);
                 }
         }
     };
 
+    const int stages = a.Kp / kCK;
     // Before stage s: A of s in LDS, B of s in slot s % 2, the loads of A of
     // s + 1 in flight in register set (s + 1) % 2.  Stage s issues B of s + 1
     // (the other slot, read last in stage s - 1) and A of s + 2 (set s % 2,
     // stored in stage s - 1), multiplies, and after a barrier waits for all
     // but the four newest loads (A of s + 2), so B of s + 1 and A of s + 1
     // have landed, and stores A of s + 1.
-    const int stages = a.Kp / kCK;
-    float4 ra0[AV], ra1[AV];
-    fetch_a(0,ra0);
-    issue_b(0,0);
-    // The image loads are issued unconditionally (past the last stage they
-    // read offsets of a further tap, in range or read as zeros, and are never
-    // stored), so every stage has the same four loads newest in the counter.
-    fetch_a(1,ra1);
-    store_a(ra0);
-    conv_barrier<4>();  // B of 0 landed (A of 1 may be in flight)
-    auto step = [&](int s, float4 (&mine)[AV], float4 (&next)[AV], int slot, bool more) {
-        if (more) issue_b(s + 1,slot ^ 1);
-        fetch_a(s + 2,mine);
-        multiply(slot);
-        if (more) {
-            conv_barrier<15>();  // every wave is done reading A of s and B slot s % 2
-            store_a(next);       // (the compiler waits for the loads of `next`)
-            conv_barrier<4>();   // B of s + 1 landed; A of s + 2 may be in flight
+    if constexpr (WIDEN) {
+        float4 ra[AV];
+        for (int s = 0; s < stages; s++) {
+            fetch_a(s,ra);
+            // 128 rows x 64 bytes, two 16-byte pieces per thread
+            cu32x4 rb[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int q = t + 256 * j;
+                rb[j] = __builtin_amdgcn_raw_buffer_load_b128(rwh,(((uint32_t)n0 + q / 4) * (uint32_t)a.Kp + 8u * (q % 4)) * 2u,
+                                                              (uint32_t)(s * kCK * 2),0);
+            }
+            __syncthreads();  // every wave is done with the stage before
+            store_a(ra);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int q = t + 256 * j, row = q / 4, at = row * 32 + (((q % 4) ^ ((row >> 2) & 3)) << 3);
+                cu32x4 hi, lo;
+                half_planes(rb[j],hi,lo);
+                *reinterpret_cast<cu32x4*>(bslot0 + at) = hi;
+                *reinterpret_cast<cu32x4*>(bslot0 + PB + at) = lo;
+            }
+            __syncthreads();
+            multiply(0);
         }
-    };
-    // Whole pairs in the loop (every step has a next stage, so the loop body
-    // has no path that leaves a register set's loads unwaited), then the
-    // last one or two stages.
-    int s = 0;
-    for (; s + 2 < stages; s += 2) {
-        step(s,ra0,ra1,0,true);
-        step(s + 1,ra1,ra0,1,true);
+    } else {
+        float4 ra0[AV], ra1[AV];
+        fetch_a(0,ra0);
+        issue_b(0,0);
+        // The image loads are issued unconditionally (past the last stage they
+        // read offsets of a further tap, in range or read as zeros, and are never
+        // stored), so every stage has the same four loads newest in the counter.
+        fetch_a(1,ra1);
+        store_a(ra0);
+        conv_barrier<4>();  // B of 0 landed (A of 1 may be in flight)
+        auto step = [&](int s, float4 (&mine)[AV], float4 (&next)[AV], int slot, bool more) {
+            if (more) issue_b(s + 1,slot ^ 1);
+            fetch_a(s + 2,mine);
+            multiply(slot);
+            if (more) {
+                conv_barrier<15>();  // every wave is done reading A of s and B slot s % 2
+                store_a(next);       // (the compiler waits for the loads of `next`)
+                conv_barrier<4>();   // B of s + 1 landed; A of s + 2 may be in flight
+            }
+        };
+        // Whole pairs in the loop (every step has a next stage, so the loop body
+        // has no path that leaves a register set's loads unwaited), then the
+        // last one or two stages.
+        int s = 0;
+        for (; s + 2 < stages; s += 2) {
+            step(s,ra0,ra1,0,true);
+            step(s + 1,ra1,ra0,1,true);
+        }
+        step(s,ra0,ra1,0,s + 1 < stages);
+        if (s + 1 < stages) step(s + 1,ra1,ra0,1,false);
     }
-    step(s,ra0,ra1,0,s + 1 < stages);
-    if (s + 1 < stages) step(s + 1,ra1,ra0,1,false);
 
+    float back = 1.0f;
+    if constexpr (HALF) {
+        // The pixels' maxima over the eight threads of each row.
+        bool out = false;
+#pragma unroll
+        for (int i = 0; i < AV; i++) {
+            float m = top[i];
+            m = __builtin_fmaxf(m,dpp_f32<kDppXor1>(m));
+            m = __builtin_fmaxf(m,dpp_f32<kDppXor2>(m));
+            m = __builtin_fmaxf(m,dpp_f32<kDppHalfMirror>(m));
+            out = out || m > 32768.0f || (m != 0.0f && m < 0.015625f);
+        }
+        if (__syncthreads_or(out)) return true;
+        back = 1.0f / scale;
+    }
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const int n = n0 + wn * 64 + 32 * j + lr;
@@ -499,14 +618,62 @@ __device__ __forceinline__ void conv_body_ring(const ConvArgs& a)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const long long m = m0 + wm * 64 + 32 * i + 8 * (r / 4) + 4 * hh + r % 4;
-                if (m < a.M) a.y[(size_t)m * a.N + n] = a.bias? __fadd_rn(acc[i][j][r],b) : acc[i][j][r];
+                const float v = HALF? acc[i][j][r] * back : acc[i][j][r];
+                if (m < a.M) a.y[(size_t)m * a.N + n] = a.bias? __fadd_rn(v,b) : v;
             }
     }
+    return false;
 }
 
+// The scale of an fp16 tile, a power of two from the largest |x| of a sample
+// (the centre tap's first 32 channels of the tile's pixels), in steps of 2^8:
+// 8 for a sample in 1/8 .. 32, so that neighbouring tiles, and the same values
+// at another place of another image, split alike.  The scaled sample is 1 ..
+// 256: the split is then fine for values up to 2^7 times the sample and for
+// pixels down to 2^-6 of it.
+__device__ __forceinline__ float conv_scale(const ConvArgs& a, uint16_t* shared)
+{
+    const int t = threadIdx.x;
+    const long long m0 = (long long)blockIdx.x * 128;
+    float most = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const long long m = m0 + t / 8 + 32 * i;
+        const int iy = (int)(m / a.OW) * a.SY - a.PT + a.KY / 2, ix = (int)(m % a.OW) * a.SX - a.PL + a.KX / 2;
+        if (m < a.M && iy >= 0 && iy < a.H && ix >= 0 && ix < a.W) {
+            const float4 v = *reinterpret_cast<const float4*>(a.x + ((size_t)iy * a.W + ix) * a.C + (t % 8) * 4);
+            most = __builtin_fmaxf(__builtin_fmaxf(most,__builtin_fabsf(v.x)),__builtin_fabsf(v.y));
+            most = __builtin_fmaxf(__builtin_fmaxf(most,__builtin_fabsf(v.z)),__builtin_fabsf(v.w));
+        }
+    }
+    most = __builtin_fmaxf(most,dpp_f32<kDppXor1>(most));
+    most = __builtin_fmaxf(most,dpp_f32<kDppXor2>(most));
+    most = __builtin_fmaxf(most,dpp_f32<kDppHalfMirror>(most));
+    most = __builtin_fmaxf(most,dpp_f32<kDppMirror>(most));
+    most = __builtin_fmaxf(__builtin_fmaxf(lane_f32(most,0),lane_f32(most,16)),__builtin_fmaxf(lane_f32(most,32),lane_f32(most,48)));
+    float* waves = reinterpret_cast<float*>(shared);
+    if ((t & 63) == 0) waves[t >> 6] = most;
+    __syncthreads();
+    most = __builtin_fmaxf(__builtin_fmaxf(waves[0],waves[1]),__builtin_fmaxf(waves[2],waves[3]));
+    __syncthreads();
+    const int e = (int)(__float_as_uint(most) >> 23);  // biased exponent: 2^(e - 127) <= most
+    const int s = e == 0 || e == 255? 130 : 130 - ((e - 124) >> 3) * 8;  // (10 .. 250)
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(s) << 23);
+}
+
+template <int FORM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3,3))) void conv_image_kernel(ConvArgs a)
 {
-    conv_body_ring(a);
+    // (separate arrays: the compiler can then tell the image stores from the
+    // transfers in flight into the ring)
+    __shared__ __attribute__((aligned(1024))) uint16_t lds[2 * 128 * kCRow];
+    __shared__ __attribute__((aligned(1024))) uint16_t bslot0[2 * kCN * 32];  // ring slots: planes hi, lo
+    __shared__ __attribute__((aligned(1024))) uint16_t bslot1[2 * kCN * 32];
+    if constexpr (FORM == kConvHalf) {
+        if (conv_body_ring<kConvHalf>(a,conv_scale(a,lds),lds,bslot0,bslot1)) conv_body_ring<kConvWiden>(a,1.0f,lds,bslot0,bslot1);
+    } else {
+        conv_body_ring<FORM>(a,1.0f,lds,bslot0,bslot1);
+    }
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3,3))) void conv_image_wide_kernel(ConvArgs a)
@@ -527,7 +694,9 @@ hipError_t launch_conv(const ConvArgs& a, hipStream_t s)
     const dim3 grid((unsigned)mt,(unsigned)(a.Npad / kCN));
     const bool narrow = (size_t)a.W * a.H * a.C * 4 < ((size_t)1 << 31) && (size_t)a.Npad * a.Kp * 2 < ((size_t)1 << 31);
     if (a.C % kCK == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0) {
-        if (narrow) conv_image_kernel<<<grid,dim3(256),0,s>>>(a);
+        if (narrow && a.kind == kConvHalf) conv_image_kernel<kConvHalf><<<grid,dim3(256),0,s>>>(a);
+        else if (narrow && a.kind == kConvBf16) conv_image_kernel<kConvBf16><<<grid,dim3(256),0,s>>>(a);
+        else if (narrow) conv_image_kernel<kConvSplit><<<grid,dim3(256),0,s>>>(a);
         else conv_image_wide_kernel<<<grid,dim3(256),0,s>>>(a);
     } else
         conv_gather_kernel<<<grid,dim3(256),0,s>>>(a);

@@ -191,9 +191,13 @@ hipError_t launch_layout(int op, const float* src, float* dst, size_t rows, size
 hipError_t launch_shortcut(const float* src, float* dst, size_t out_rows, size_t channels, size_t src_channels, size_t width, size_t side,
                            size_t temporal, bool up, hipStream_t s);
 
-// conv.hip: implicit-GEMM convolution on split-bf16 MFMA.  The weight form is
-// two bf16 planes [Npad][Kp] (hi, lo) with the inner index in (ky, kx, c)
-// order; x [H*W][C], y [OH*OW][N] (+ bias[n] when bias is not null).
+// conv.hip: implicit-GEMM convolution on MFMA.  The weight form is one or two
+// 16-bit planes [Npad][Kp] with the inner index in (ky, kx, c) order; x
+// [H*W][C], y [OH*OW][N] (+ bias[n] when bias is not null).
+constexpr int kConvSplit = 0;  // two bf16 planes, hi and lo
+constexpr int kConvBf16 = 1;   // one bf16 plane (BF16 weights)
+constexpr int kConvHalf = 2;   // one fp16 plane (F16 weights)
+int conv_weight_kind(uint32_t type, int cin);
 struct ConvArgs {
     const float* x;
     const uint16_t *wh, *wl;
@@ -201,9 +205,10 @@ struct ConvArgs {
     float* y;
     int W, H, C, KX, KY, SX, SY, PL, PT, OW, OH, K, Kp, N, Npad;
     long long M;
+    int kind;  // the weight's form; wl is read for kConvSplit only
 };
 constexpr int kConvTileN = 128, kConvTileK = 32;
-hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad,
+hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad, int kind,
                             uint16_t* hi, uint16_t* lo, hipStream_t s);
 hipError_t launch_conv(const ConvArgs& a, hipStream_t s);
 

@@ -96,6 +96,34 @@ def test_against_oracle(sess, wd, ht, cin, cout, k, wtype, geom, bias):
     assert err <= TOL
 
 
+@pytest.mark.parametrize("scale", ["1e-30", "1e-3", "1e5", "1e30", "mixed", "zeros"])
+@pytest.mark.parametrize("geom", [None, (2, 2, 0, 1, 0, 1)])
+def test_half_weights_over_the_range(sess, scale, geom):
+    """F16 weights multiply the image split in fp16 under a power-of-two scale
+    per tile: image values over fp32's range, pixels of very different
+    magnitude next to each other (those tiles run the bf16 products), zeros.
+    Held to the bf16 split's own bound per output: 3 * 2^-17 of the largest
+    |x| * sum |w|, the worst case of one output's terms adding up."""
+    rng = np.random.default_rng(7)
+    wd, ht, cin, cout, k = 37, 21, 64, 72, 3
+    x = rng.standard_normal((wd * ht, cin)).astype(np.float32)
+    if scale == "mixed":
+        x *= (10.0 ** rng.uniform(-12, 8, (wd * ht, 1))).astype(np.float32)
+    elif scale == "zeros":
+        x[rng.random(wd * ht) < 0.7] = 0
+        x[: 6 * wd] = 0
+    else:
+        x *= np.float32(scale)
+    w = (rng.standard_normal((cout, cin * k * k)) / np.sqrt(cin * k * k)).astype(np.float32)
+    raw, wv = weight_bytes(w, F16)
+    y = gpu_conv(sess, f"conv:half:{scale}", x, wd, ht, raw, F16, k, k, cin, cout, None, geom)
+    ref = conv2d(oracle(), x, wd, ht, wv, k, k, None, geom)
+    top = conv2d(oracle(), np.abs(x), wd, ht, np.abs(wv), k, k, None, geom)  # sum |x| |w| of each output
+    peak = top.max(axis=1, keepdims=True)
+    assert np.all(np.abs(y - ref) <= 3 * 2.0 ** -17 * peak + 1e-37), float((np.abs(y - ref) / np.maximum(peak, 1e-37)).max())
+    assert np.all(y[peak[:, 0] == 0] == 0)
+
+
 def test_vae_shape_band_and_translation(sess):
     """256 x 256 pixels, 512 -> 512 channels, 3x3 (a VAE decoder block's
     conv): output rows 0-1 and 127-128 against the oracle run on the input
