@@ -1991,7 +1991,17 @@ int pixhip_conv2d(pixhip_session* s, const pixhip_weight* wc, const float* input
     a.N = (int)w->rows;
     a.Npad = (int)w->conv_npad;
     a.M = (long long)(ow * oh);
-    hipError_t e = pixhip::launch_conv(a,s->stream);
+    // The workspace of a split inner range is wanted, not needed: without it
+    // (no memory, or the stream is being captured, when nothing may be
+    // allocated) the call runs whole.
+    int pieces = pixhip::conv_pieces(a);
+    const size_t part_bytes = (size_t)pieces * out_bytes;
+    if (pieces > 1 && part_bytes > s->partial_bytes) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s->stream,&capture) != hipSuccess) (void)hipGetLastError();
+        if (capture != hipStreamCaptureStatusNone || grow(s,&s->partial,&s->partial_bytes,part_bytes)) pieces = 1;
+    }
+    hipError_t e = pixhip::launch_conv(a,pieces,pieces > 1? static_cast<float*>(s->partial) : nullptr,s->stream);
     if (e == hipErrorInvalidValue) return fail(PIXHIP_ERR_ARGUMENT,"convolution grid too large");
     PIX_HIP(e,"convolution");
     return PIXHIP_OK;

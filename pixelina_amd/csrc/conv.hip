@@ -425,6 +425,9 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
             ix0[i] = 0;
         }
     }
+    // (stages counted from this piece's first: the whole inner range unless split)
+    const int first = a.part? (int)blockIdx.z * a.piece_stages : 0;
+    const int stages = a.part? min(a.piece_stages,a.Kp / kCK - first) : a.Kp / kCK;
     const uint32_t wbytes = (uint32_t)((size_t)a.Npad * a.Kp * 2);
     const CRsrc rx = conv_rsrc(a.x,(uint32_t)((size_t)a.W * a.H * a.C * 4));
     const CRsrc rwh = conv_rsrc(a.wh,wbytes), rwl = conv_rsrc(FORM == kConvSplit? a.wl : a.wh,wbytes);
@@ -441,14 +444,14 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
         for (int i = 0; i < CHUNKS; i++) {
             const int c = wave + 4 * i;
             uint16_t* dst = (slot? bslot1 : bslot0) + (c / 8) * PB + (c % 8) * 512;
-            conv_dma(c < 8? rwh : rwl,dst,bvo[i],(uint32_t)(stage * kCK * 2));
+            conv_dma(c < 8? rwh : rwl,dst,bvo[i],(uint32_t)((first + stage) * kCK * 2));
         }
     };
     constexpr uint32_t kOut = 0x80000000u;
     uint32_t aoff[AV];
     int cur_tap = -1;
     auto fetch_a = [&](int stage, float4 (&ra)[AV]) {
-        const int k0 = stage * kCK, tap = k0 / a.C;
+        const int k0 = (first + stage) * kCK, tap = k0 / a.C;
         if (tap != cur_tap) {
             cur_tap = tap;
             const int ky = tap / a.KX, kx = tap % a.KX;
@@ -529,7 +532,6 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
         }
     };
 
-    const int stages = a.Kp / kCK;
     // Before stage s: A of s in LDS, B of s in slot s % 2, the loads of A of
     // s + 1 in flight in register set (s + 1) % 2.  Stage s issues B of s + 1
     // (the other slot, read last in stage s - 1) and A of s + 2 (set s % 2,
@@ -546,7 +548,7 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
             for (int j = 0; j < 2; j++) {
                 const int q = t + 256 * j;
                 rb[j] = __builtin_amdgcn_raw_buffer_load_b128(rwh,(((uint32_t)n0 + q / 4) * (uint32_t)a.Kp + 8u * (q % 4)) * 2u,
-                                                              (uint32_t)(s * kCK * 2),0);
+                                                              (uint32_t)((first + s) * kCK * 2),0);
             }
             __syncthreads();  // every wave is done with the stage before
             store_a(ra);
@@ -593,33 +595,36 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
         if (s + 1 < stages) step(s + 1,ra1,ra0,1,false);
     }
 
+    // A piece leaves its sums to conv_reduce_kernel, which adds the bias.
+    float* const out = a.part? a.part + (size_t)blockIdx.z * (size_t)a.M * a.N : a.y;
+    const float* const bias = a.part? nullptr : a.bias;
     float back = 1.0f;
     if constexpr (HALF) {
         // The pixels' maxima over the eight threads of each row.
-        bool out = false;
+        bool outside = false;
 #pragma unroll
         for (int i = 0; i < AV; i++) {
             float m = top[i];
             m = __builtin_fmaxf(m,dpp_f32<kDppXor1>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppXor2>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppHalfMirror>(m));
-            out = out || m > 32768.0f || (m != 0.0f && m < 0.015625f);
+            outside = outside || m > 32768.0f || (m != 0.0f && m < 0.015625f);
         }
-        if (__syncthreads_or(out)) return true;
+        if (__syncthreads_or(outside)) return true;
         back = 1.0f / scale;
     }
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const int n = n0 + wn * 64 + 32 * j + lr;
         if (n >= a.N) continue;
-        const float b = a.bias? a.bias[n] : 0.0f;
+        const float b = bias? bias[n] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const long long m = m0 + wm * 64 + 32 * i + 8 * (r / 4) + 4 * hh + r % 4;
                 const float v = HALF? acc[i][j][r] * back : acc[i][j][r];
-                if (m < a.M) a.y[(size_t)m * a.N + n] = a.bias? __fadd_rn(v,b) : v;
+                if (m < a.M) out[(size_t)m * a.N + n] = bias? __fadd_rn(v,b) : v;
             }
     }
     return false;
@@ -686,20 +691,79 @@ __global__ __launch_bounds__(256) void conv_gather_kernel(ConvArgs a)
     conv_body<0>(a);
 }
 
-hipError_t launch_conv(const ConvArgs& a, hipStream_t s)
+// y = the pieces' sums, in order, + bias.
+__global__ __launch_bounds__(256) void conv_reduce_kernel(const float* __restrict__ part, int pieces, size_t total, int N, const float* bias,
+                                                          float* __restrict__ y)
 {
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) return;
+    float v = part[e];
+    for (int p = 1; p < pieces; p++) v += part[(size_t)p * total + e];
+    y[e] = bias? __fadd_rn(v,bias[e % (unsigned)N]) : v;
+}
+
+// Whether a call runs the image kernel (a stage is whole channels, 32-bit offsets).
+static bool image_form(const ConvArgs& a)
+{
+    const size_t lim = (size_t)1 << 31;
+    return a.C % kCK == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && (size_t)a.W * a.H * a.C * 4 < lim &&
+           (size_t)a.Npad * a.Kp * 2 < lim;
+}
+
+// Pieces of the inner range for images whose tiles leave CUs idle (one: none).
+// A workgroup alone on a CU takes about 0.78 us a stage, several together 0.62
+// each; pieces cost about 8 us more and a pass that moves (pieces + 1) fp32
+// images at about 4 TB/s.  The estimate's least is taken.  Measured, us, whole /
+// the pieces taken (F16 weights, 3x3): 40^2 pixels 512 -> 512 (52 tiles) 117.8 /
+// 43, 64^2 (128 tiles) 118 / 66, 200 x 100 128 -> 3 (157 tiles) 36.5 / 24.5,
+// 90^2 384 -> 384 (192 tiles) 92 / 74, 128^2 512 -> 256 (256 tiles) 120 / 112;
+// 1x1 at 30^2 (16 stages) gains nothing and stays whole.
+int conv_pieces(const ConvArgs& a)
+{
+    const long long tiles = (a.M + 127) / 128 * (a.Npad / kCN), cus = device_cus();
+    const int stages = a.Kp / kCK;
+    if (!image_form(a) || tiles > cus) return 1;
+    int best = 1;
+    double least = 0.78 * stages;
+    for (int p = 2; p <= stages / 4 && p * tiles <= 3 * cus; p++) {
+        const int length = (stages + p - 1) / p;
+        if ((stages + length - 1) / length != p) continue;  // an empty last piece
+        const long long rounds = (p * tiles + cus - 1) / cus;
+        const double t = length * (rounds == 1? 0.78 : 0.62 * rounds) + 8.0 + (p + 1) * (double)a.M * a.N * 4.0 / 4e6;
+        if (t < least) {
+            least = t;
+            best = p;
+        }
+    }
+    return best;
+}
+
+hipError_t launch_conv(const ConvArgs& args, int pieces, float* part, hipStream_t s)
+{
+    ConvArgs a = args;
     if (!a.M || !a.N) return hipSuccess;
     const long long mt = (a.M + 127) / 128;
     if (mt > 0x7fffffffLL || a.Npad / kCN > 65535) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)mt,(unsigned)(a.Npad / kCN));
-    const bool narrow = (size_t)a.W * a.H * a.C * 4 < ((size_t)1 << 31) && (size_t)a.Npad * a.Kp * 2 < ((size_t)1 << 31);
-    if (a.C % kCK == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0) {
-        if (narrow && a.kind == kConvHalf) conv_image_kernel<kConvHalf><<<grid,dim3(256),0,s>>>(a);
-        else if (narrow && a.kind == kConvBf16) conv_image_kernel<kConvBf16><<<grid,dim3(256),0,s>>>(a);
-        else if (narrow) conv_image_kernel<kConvSplit><<<grid,dim3(256),0,s>>>(a);
-        else conv_image_wide_kernel<<<grid,dim3(256),0,s>>>(a);
-    } else
+    if (pieces > 1 && part) {
+        a.part = part;
+        a.piece_stages = (a.Kp / kCK + pieces - 1) / pieces;
+    }
+    const dim3 grid((unsigned)mt,(unsigned)(a.Npad / kCN),a.part? (unsigned)pieces : 1u);
+    if (image_form(a)) {
+        if (a.kind == kConvHalf) conv_image_kernel<kConvHalf><<<grid,dim3(256),0,s>>>(a);
+        else if (a.kind == kConvBf16) conv_image_kernel<kConvBf16><<<grid,dim3(256),0,s>>>(a);
+        else conv_image_kernel<kConvSplit><<<grid,dim3(256),0,s>>>(a);
+    } else if (a.C % kCK == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0) {
+        conv_image_wide_kernel<<<grid,dim3(256),0,s>>>(a);
+    } else {
         conv_gather_kernel<<<grid,dim3(256),0,s>>>(a);
+    }
+    if (a.part) {
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        const size_t total = (size_t)a.M * a.N;
+        conv_reduce_kernel<<<dim3((unsigned)((total + 255) / 256)),dim3(256),0,s>>>(part,pieces,total,a.N,a.bias,a.y);
+    }
     return hipGetLastError();
 }
 

@@ -206,11 +206,16 @@ struct ConvArgs {
     int W, H, C, KX, KY, SX, SY, PL, PT, OW, OH, K, Kp, N, Npad;
     long long M;
     int kind;  // the weight's form; wl is read for kConvSplit only
+    float* part;       // pieces of the inner range: their sums [piece][M][N] (launch_conv sets both)
+    int piece_stages;
 };
 constexpr int kConvTileN = 128, kConvTileK = 32;
 hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad, int kind,
                             uint16_t* hi, uint16_t* lo, hipStream_t s);
-hipError_t launch_conv(const ConvArgs& a, hipStream_t s);
+// Pieces of the inner range a call is worth cutting into (1: none); launch_conv
+// takes a workspace of pieces * M * N floats for them, or null to run whole.
+int conv_pieces(const ConvArgs& a);
+hipError_t launch_conv(const ConvArgs& a, int pieces, float* part, hipStream_t s);
 
 // repack.hip
 hipError_t launch_repack_q5_K(const uint8_t* raw, size_t rows, size_t inner, size_t npad, int8_t* hi, int8_t* lo, float* d,

@@ -81,6 +81,10 @@ def test_reference_vectors(sess):
     (19, 13, 32, 160, 1, F16, None, True),              # one 32-value stage (the pipelined kernel's tail alone)
     (17, 11, 64, 96, 1, BF16, None, False),             # two stages
     (23, 9, 96, 128, 1, F32, None, True),               # three stages
+    (40, 24, 512, 200, 3, F16, None, True),             # inner range in pieces, added by the reduction
+    (31, 29, 288, 130, 3, BF16, None, False),           # pieces, the last one shorter
+    (65, 33, 160, 3, 3, F32, (2, 2, 0, 1, 0, 1), True),
+    (128, 127, 128, 128, 3, F16, None, True),           # 127 tiles
 ])
 def test_against_oracle(sess, wd, ht, cin, cout, k, wtype, geom, bias):
     rng = np.random.default_rng(wd * cin + cout)
