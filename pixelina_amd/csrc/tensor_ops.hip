@@ -376,21 +376,22 @@ struct GnStat {
     float pad;
 };
 
-// One non-temporal load of VEC floats at byte offset `off` of a raw buffer
-// (zeros past its end).
-template <int VEC> __device__ __forceinline__ typename Vec<VEC>::T nt_buffer_load(__amdgpu_buffer_rsrc_t r, int off)
+// One load of VEC floats at byte offset `off` of a raw buffer (zeros past its
+// end), non-temporal or (KEEP) plain.
+template <int VEC, bool KEEP> __device__ __forceinline__ typename Vec<VEC>::T gn_buffer_load(__amdgpu_buffer_rsrc_t r, int off)
 {
+    constexpr int AUX = KEEP? 0 : 2;
     if constexpr (VEC == 4) {
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-        const u32x4 u = __builtin_amdgcn_raw_buffer_load_b128(r,off,0,2);
+        const u32x4 u = __builtin_amdgcn_raw_buffer_load_b128(r,off,0,AUX);
         return make_float4(__uint_as_float(u.x),__uint_as_float(u.y),__uint_as_float(u.z),__uint_as_float(u.w));
     } else {
-        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r,off,0,2));
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r,off,0,AUX));
     }
 }
 
 template <int VEC>
-__global__ __launch_bounds__(256) void gn_partial_kernel(const float* __restrict__ x, GnShape sh, double* __restrict__ part)
+__global__ __launch_bounds__(256) void gn_partial_kernel(const float* __restrict__ x, GnShape sh, size_t keep_row, double* __restrict__ part)
 {
     typedef typename Vec<VEC>::T T;
     __shared__ double red[256];
@@ -414,7 +415,8 @@ __global__ __launch_bounds__(256) void gn_partial_kernel(const float* __restrict
     if (active) {
         // all loads first, then the sums (rows past the end add zero)
 #pragma unroll
-        for (int k = 0; k < kGnRows; k++) v[k] = nt_buffer_load<VEC>(rx,first + k * pitch);
+        for (int k = 0; k < kGnRows; k++)
+            v[k] = row0 >= keep_row? gn_buffer_load<VEC,true>(rx,first + k * pitch) : gn_buffer_load<VEC,false>(rx,first + k * pitch);
 #pragma unroll
         for (int k = 0; k < kGnRows; k++)
 #pragma unroll
@@ -545,10 +547,13 @@ __global__ __launch_bounds__(256) void gn_merge_kernel(const double* __restrict_
 }
 
 // With FIXED (256 a multiple of cvec) every value of a thread lies in one
-// column, whose weight, bias and group statistics are read once.
+// column, whose weight, bias and group statistics are read once.  Spans run from
+// the last to the first: rows from keep_row on were left in the last-level cache
+// by the statistics pass.
 template <int VEC, bool FIXED, bool NT>
 __global__ __launch_bounds__(256) void gn_apply_kernel(const float* __restrict__ x, GnShape sh, const GnStat* __restrict__ stat,
-                                                       const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y)
+                                                       const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y,
+                                                       size_t keep_row)
 {
     typedef typename Vec<VEC>::T T;
     __shared__ GnStat st[kGroups];
@@ -567,12 +572,19 @@ __global__ __launch_bounds__(256) void gn_apply_kernel(const float* __restrict__
             bf[j] = b[c + j];
         }
     }
-    for (size_t p = blockIdx.x; p < spans; p += gridDim.x) {
-        const size_t base = p * span + threadIdx.x;
+    const size_t keep = keep_row * sh.cvec;
+    for (size_t r = blockIdx.x; r < spans; r += gridDim.x) {
+        const size_t p = spans - 1 - r, base = p * span + threadIdx.x;
         T v[kUnroll];
+        if (p * span >= keep) {
 #pragma unroll
-        for (int k = 0; k < kUnroll; k++)
-            if (base + k * (size_t)blockDim.x < total) v[k] = nt_load(reinterpret_cast<const T*>(x + (base + k * (size_t)blockDim.x) * VEC));
+            for (int k = 0; k < kUnroll; k++)
+                if (base + k * (size_t)blockDim.x < total) v[k] = *reinterpret_cast<const T*>(x + (base + k * (size_t)blockDim.x) * VEC);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kUnroll; k++)
+                if (base + k * (size_t)blockDim.x < total) v[k] = nt_load(reinterpret_cast<const T*>(x + (base + k * (size_t)blockDim.x) * VEC));
+        }
 #pragma unroll
         for (int k = 0; k < kUnroll; k++) {
             const size_t e = base + k * (size_t)blockDim.x;
@@ -638,8 +650,19 @@ hipError_t launch_groupnorm(const float* x, const float* w, const float* b, floa
     double* level = reinterpret_cast<double*>(stat + kGroups);
     double* part = level + kGroups * kGnSplit * 3;
     const dim3 pgrid((unsigned)sh.chunks,(unsigned)sh.tiles), block(256);
-    if (vec) gn_partial_kernel<4><<<pgrid,block,0,s>>>(x,sh,part);
-    else gn_partial_kernel<1><<<pgrid,block,0,s>>>(x,sh,part);
+    // The rows the apply pass finds in the last-level cache: it runs from the last
+    // row down, and the statistics pass reads the last 224 MB with plain loads, the
+    // rows before them past the caches.  Us a call, everything past the caches /
+    // so: [1M, 128] 270 / 252, [256K, 512] 277 / 253, [1M, 96] 370 / 308.  Between
+    // 64 and 256 MB (plain output stores) wide rows lose, the output pushes the
+    // input out: [256K, 128] 82 / 90, [256K, 256] 147 / 158; rows below 512 bytes
+    // gain at every size ([340K, 96] 138 / 110, [500K, 64] 101 / 90).
+    const size_t bytes = rows * channels * sizeof(float);
+    const bool keep = channels < 128 || bytes > kStreamBytes || bytes <= ((size_t)64 << 20);
+    const size_t kept = keep? ((size_t)224 << 20) / (channels * sizeof(float)) : 0;
+    const size_t keep_row = rows > kept? rows - kept : 0;
+    if (vec) gn_partial_kernel<4><<<pgrid,block,0,s>>>(x,sh,keep_row,part);
+    else gn_partial_kernel<1><<<pgrid,block,0,s>>>(x,sh,keep_row,part);
     // at least 1024 chunks per first-level block
     const unsigned split = (unsigned)std::min<size_t>(kGnSplit,std::max<size_t>(1,(sh.chunks + 1023) / 1024));
     gn_merge_kernel<true><<<dim3(kGroups,split),block,0,s>>>(part,sh.chunks,sh,eps,level,stat);
@@ -648,10 +671,10 @@ hipError_t launch_groupnorm(const float* x, const float* w, const float* b, floa
     const bool fixed = 256 % sh.cvec == 0;
     auto apply = [&](auto nt) {
         constexpr bool NT = decltype(nt)::value;
-        if (vec && fixed) gn_apply_kernel<4,true,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y);
-        else if (vec) gn_apply_kernel<4,false,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y);
-        else if (fixed) gn_apply_kernel<1,true,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y);
-        else gn_apply_kernel<1,false,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y);
+        if (vec && fixed) gn_apply_kernel<4,true,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+        else if (vec) gn_apply_kernel<4,false,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+        else if (fixed) gn_apply_kernel<1,true,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+        else gn_apply_kernel<1,false,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
     };
     if (rows * channels * sizeof(float) > kStreamBytes) apply(std::true_type());
     else apply(std::false_type());
