@@ -94,7 +94,7 @@ __device__ __forceinline__ void store_chunk(const FuseArgs& a, size_t row, int c
         quantize_q8_0_group(v,packed,d32,dh);
         const size_t b = (size_t)c * 8 + (lane >> 3), nb = K / PIX_QK8, nbp = a.kpad / PIX_QK8;
         if (a.qs && b < nbp) {
-            reinterpret_cast<uint32_t*>(a.qs + row * a.kpad + b * PIX_QK8)[lane & 7] = packed;
+            *reinterpret_cast<uint32_t*>(a.qs + tiled_offset(row,b * PIX_QK8 + 4 * (lane & 7),a.kpad)) = packed;
             if ((lane & 7) == 0) a.d[b * a.mpad + row] = half_bits_to_float(dh);
         }
         if (a.blocks && b < nb) {

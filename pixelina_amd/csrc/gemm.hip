@@ -20,8 +20,8 @@
 //
 // Data movement: K advances in 64-value stages (two blocks), loaded with
 // buffer_load_dwordx4 ... lds (HBM -> LDS, no registers) into a 4-stage ring.
-// Lane l of a DMA lands at LDS base + 16*l; four consecutive lanes fetch one
-// 64-byte row (coalesced), each lane picking its piece so that the ring holds
+// Lane l of a DMA lands at LDS base + 16*l; a DMA reads one contiguous 1 KB
+// piece of a tiled plane (16 rows x 64 values), each lane picking its piece so that the ring holds
 // rows of four 16-byte pieces with piece c of row r at slot 4r + (c ^ ((r>>2)
 // & 3)): the MFMA operand reads (ds_read_b128, lane l reads row l%32, piece
 // 2s + l/32) are then free of LDS bank conflicts.  Each stage's block scales
@@ -65,9 +65,9 @@ constexpr int kSlotXd80 = 512, kSlotWd80 = 640;
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 
 struct GemmArgs {
-    const int8_t* xq;     // [Mpad][K]
+    const int8_t* xq;     // tiled [Mpad/16][K/64][16][64]
     const float* xdT;     // [K/32][Mpad]
-    const int8_t* wq;     // [Npad][K]
+    const int8_t* wq;     // tiled [Npad/16][K/64][16][64]
     const float* wdT;     // [K/32][Npad]
     float* y;
     const float* bias;
@@ -163,7 +163,7 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks)
 // l/4, piece (l%4) ^ ((l/16) & 3).
 __device__ __forceinline__ void issue_stage(const GemmArgs& g, const Ctx& x, int c, uint8_t* sa, uint8_t* sw, uint8_t* discard)
 {
-    const uint32_t k0 = (uint32_t)c * kKC;
+    const uint32_t k0 = (uint32_t)c * 1024u;  // stage c of a row group's tiled plane
     uint32_t vo_rows = 0;  // per-lane source offset of a 64-B row piece (for the row chunks)
 #pragma unroll
     for (int q = 0; q < kPerWave; q++) {
@@ -171,7 +171,7 @@ __device__ __forceinline__ void issue_stage(const GemmArgs& g, const Ctx& x, int
         uint8_t* dst = chunk < 16? sa + chunk * kChunk : sw + (chunk - 16) * kChunk;
         if (chunk < 24) {
             const uint32_t lane = lane_now();
-            vo_rows = (lane >> 2) * (uint32_t)x.K + 16u * ((lane & 3) ^ ((lane >> 4) & 3));
+            vo_rows = 16u * ((lane & ~3u) | ((lane & 3) ^ ((lane >> 4) & 3)));
         }
         if (chunk < 16) {
             dma(x.rx,dst,vo_rows,(uint32_t)(x.m0 + chunk * 16) * x.K + k0);
@@ -323,7 +323,7 @@ __device__ __forceinline__ Lanes lanes_of(const GemmArgs& g, const Ctx& x)
     }
     L.sx = kWRing + (hi? kZero : 16 * kSlotXd80 + (x.wm * 64 + lr) * 4);
     L.sw = kWRing + (hi? kZero : 16 * kSlotWd80 + (x.wn * kWN + lr) * 4);
-    const uint32_t rows = (ln >> 2) * (uint32_t)x.K + 16u * ((ln & 3) ^ ((ln >> 4) & 3));
+    const uint32_t rows = 16u * ((ln & ~3u) | ((ln & 3) ^ ((ln >> 4) & 3)));
     L.d0 = rows;  // chunk x.wave < 16: activation rows
     const int c1 = x.wave + kWaves;
     L.d1 = c1 < 24? rows : c1 < 26? 16u * ln : c1 == 26? 16u * lr + hi * 4u * (uint32_t)g.Npad : 0u;
@@ -334,7 +334,7 @@ __device__ __forceinline__ Lanes lanes_of(const GemmArgs& g, const Ctx& x)
 template <int SLOT>
 __device__ __forceinline__ void issue_slot(const GemmArgs& g, const Ctx& x, const Lanes& L, int c, uint8_t* lds)
 {
-    const uint32_t k0 = (uint32_t)c * kKC;
+    const uint32_t k0 = (uint32_t)c * 1024u;  // stage c of a row group's tiled plane
     uint8_t* sa = lds + SLOT * kHalfBytes;
     uint8_t* sw = lds + kWRing + SLOT * kHalfBytes;
     const int c0 = x.wave, c1 = x.wave + kWaves;
@@ -596,7 +596,7 @@ __device__ __forceinline__ SmallLanes small_lanes(const SmallCtx& x, uint32_t ri
     }
     L.sx = ring + (hi? kSZero : kSXd + (x.wm * 32 + lr) * 4);
     L.sw = ring + (hi? kSZero : kSWd + (x.wn * 32 + lr) * 4);
-    L.d_rows = (ln >> 2) * (uint32_t)x.K + 16u * ((ln & 3) ^ ((ln >> 4) & 3));
+    L.d_rows = 16u * ((ln & ~3u) | ((ln & 3) ^ ((ln >> 4) & 3)));
     L.d_scale = 4u * ln;
     return L;
 }
@@ -607,7 +607,7 @@ __device__ __forceinline__ SmallLanes small_lanes(const SmallCtx& x, uint32_t ri
 template <int SLOT>
 __device__ __forceinline__ void small_issue(const SmallCtx& x, const SmallLanes& L, int c, uint8_t* ring)
 {
-    const uint32_t k0 = (uint32_t)c * kKC;
+    const uint32_t k0 = (uint32_t)c * 1024u;  // stage c of a row group's tiled plane
     uint8_t* slot = ring + SLOT * kSSlotBytes;
     dma(x.rx,slot + x.q * kChunk,L.d_rows,(uint32_t)(x.m0 + x.q * 16) * x.K + k0);
     dma(x.rwq,slot + (x.q + 4) * kChunk,L.d_rows,(uint32_t)(x.n0 + x.q * 16) * x.K + k0);

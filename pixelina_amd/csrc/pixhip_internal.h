@@ -14,7 +14,7 @@
 //                 block; within a row the order is 0,2,..,14,1,3,..,15 (even groups,
 //                 then odd: the min-term MFMA operand order)
 //   activations, Q8_0 ("act80"), rows of Kp = K rounded up to 64 (a zero pad block):
-//     qs   int8   [M][Kp]
+//     qs   int8   tiled [Mpad/16][Kp/64][16][64] (tiled_offset)
 //     d    fp32   [Kp/32][Mpad]   fp16-rounded block scale widened to fp32
 //   Activations are allocated with Mpad rows (multiple of PIX_GEMM_MTILE) and
 //   GEMM weight forms with Npad rows (multiple of PIX_GEMM_NTILE).
@@ -26,7 +26,7 @@
 //     mn   fp16   [K/256][Npad][8]  the eight six-bit sub-block minima
 //   weights Q6_K for the GEMM: hi/lo of scale*(q-32) = 64*hi + lo (tiled as Q5_K), d fp32 [K/256][Npad]
 //   weights Q8_0 for the GEMM, rows of Kp with a zero pad block: qs int8
-//     [Npad][Kp], and the scales widened and transposed, dT fp32 [Kp/32][Npad]
+//     tiled [Npad/16][Kp/64][16][64], and the scales widened and transposed, dT fp32 [Kp/32][Npad]
 //   weights Q8_0 for the matvec: qs_mv int8 [N][4][Kp/64][16] (each row
 //     piece-major: 16-byte piece p of 64-value unit u at (p*Kp/64 + u)*16),
 //     d fp16 [N][Kp/32]
@@ -93,7 +93,7 @@ struct Act8K {
 };
 
 struct Act80 {
-    int8_t* qs;       // [mpad][Kp]
+    int8_t* qs;       // tiled [mpad/16][Kp/64][16][64]
     float* d;         // [Kp/32][mpad]
     size_t mpad;
 };
@@ -115,7 +115,7 @@ struct PlanesQ6K {
 };
 
 struct PlanarQ80 {
-    const int8_t* qs;     // [Npad][Kp] (GEMM)
+    const int8_t* qs;     // tiled [Npad/16][Kp/64][16][64] (GEMM)
     const float* dT;      // [Kp/32][Npad] (GEMM)
     const int8_t* qs_mv;  // [N][4][Kp/64][16]: each row piece-major (matvec)
     const _Float16* d;    // [N][Kp/32] (matvec)

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * kQuantWaves) void quantize_q8_0_kernel(const f
         uint16_t dh;
         quantize_q8_0_group(v[i],packed,d32,dh);
         if (qs && b < nbp) {
-            reinterpret_cast<uint32_t*>(qs + row * kpad + (size_t)b * PIX_QK8)[lane & 7] = packed;
+            *reinterpret_cast<uint32_t*>(qs + tiled_offset(row,(size_t)b * PIX_QK8 + 4 * (lane & 7),kpad)) = packed;
             if ((lane & 7) == 0) dT[(size_t)b * mpad + row] = half_bits_to_float(dh);
         }
         if (blocks && real) {

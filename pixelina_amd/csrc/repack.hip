@@ -150,7 +150,7 @@ __global__ __launch_bounds__(256) void repack_q8_0_kernel(const uint8_t* __restr
     uint32_t v = (uint32_t)s16[0] | ((uint32_t)s16[1] << 16);
     const uint16_t h = *reinterpret_cast<const uint16_t*>(src);
     if (qs) {
-        *reinterpret_cast<uint32_t*>(qs + row * kpad + b * PIX_QK8 + 4 * part) = v;
+        *reinterpret_cast<uint32_t*>(qs + tiled_offset(row,b * PIX_QK8 + 4 * part,kpad)) = v;
         if (part == 0) dT[b * rows_pad + row] = half_bits_to_float(h);
     }
     if (qs_mv) {
