@@ -20,6 +20,7 @@ SOURCES = [
     "csrc/gemm.hip",
     "csrc/gemm_kq.hip",
     "csrc/gemm_kq_rows.hip",
+    "csrc/gemm_q8_rows.hip",
     "csrc/matvec.hip",
     "csrc/fuse.hip",
     "csrc/ops.hip",
@@ -78,6 +79,7 @@ NO_SPILL = {
                            "attn_wide_kernelILi64E"),
     "csrc/gemm_kq.hip": ("gemm_kq_kernelILb1ELb0E", "gemm_kq_kernelILb0ELb0E"),
     "csrc/gemm_kq_rows.hip": ("gemm_kq_rows_kernel",),
+    "csrc/gemm_q8_rows.hip": ("gemm_q8_rows_kernel",),
     "csrc/gemm.hip": ("gemm_kernelILb0E", "gemm_small_kernel"),
 }
 

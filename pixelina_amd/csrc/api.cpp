@@ -579,7 +579,7 @@ int multiply_stage(pixhip_session* s, pixhip_weight* w, size_t columns, const pi
         return fail(PIXHIP_ERR_STATE,"no quantized activations of this shape: run the QUANTIZE stage first");
     int rc = ensure_gemm_form(s,w);
     if (rc) return rc;
-    const bool few = kind == 1 && pixhip::gemm_kq_rows(columns,w->rows,w->inner);
+    const bool few = kind == 1? pixhip::gemm_kq_rows(columns,w->rows,w->inner) : pixhip::gemm_q8_rows(columns,w->rows,w->inner);
     const size_t part_bytes = few || (kind == 2 && pixhip::gemm_q8_0_grouped(columns,w->rows))
                                   ? 0
                                   : pixhip::gemm_split_bytes(columns,w->rows,round_up(w->inner,64));
@@ -590,6 +590,7 @@ int multiply_stage(pixhip_session* s, pixhip_weight* w, size_t columns, const pi
     float* part = part_bytes? static_cast<float*>(s->partial) : nullptr;
     hipError_t e;
     if (few && w->type == PIX_Q5_K) e = pixhip::launch_gemm_rows_q5_K(s->a8k,w->q5,columns,w->rows,w->inner,out,s->stream);
+    else if (few && kind == 2) e = pixhip::launch_gemm_rows_q8_0(s->a80,w->q80,columns,w->rows,w->inner,out,s->stream);
     else if (few) e = pixhip::launch_gemm_rows_q6_K(s->a8k,w->q6,columns,w->rows,w->inner,out,s->stream);
     else if (w->type == PIX_Q5_K) e = pixhip::launch_gemm_q5_K(s->a8k,w->q5,columns,w->rows,w->inner,out,part,s->stream);
     else if (w->type == PIX_Q6_K) e = pixhip::launch_gemm_q6_K(s->a8k,w->q6,columns,w->rows,w->inner,out,part,s->stream);
@@ -686,7 +687,9 @@ int run_pipelined(pixhip_session* s, pixhip_weight* w, const float* input, size_
             const size_t kp = round_up(K,64);
             const pixhip::Act80 a = {s->a80.qs + r0 * kp,s->a80.d + r0,s->a80.mpad};
             PIX_HIP(pixhip::launch_quantize_q8_0(xs + r0 * K,rows,K,kp,a,nullptr,s->stream),"quantize Q8_0");
-            e = pixhip::launch_gemm_q8_0(a,w->q80,rows,N,K,out,part,s->stream);
+            // (the few-token form's bits do not depend on the rows of a call)
+            e = pixhip::gemm_q8_rows(columns,N,K)? pixhip::launch_gemm_rows_q8_0(a,w->q80,rows,N,K,out,s->stream)
+                                                 : pixhip::launch_gemm_q8_0(a,w->q80,rows,N,K,out,part,s->stream);
         } else {
             // tiled planes: rows r0.. (r0 a multiple of 32) start r0*K bytes in, the
             // 16-value sums r0*K/16 elements in; the scales r0 columns in
@@ -1144,7 +1147,8 @@ int pixhip_matmul_ex_noalloc(pixhip_session* s, const pixhip_weight* wc, const f
                                               std::to_string(c.offset) + " bytes, beyond the 32 MiB allocation-free scratch");
         const pixhip::Act80 a = {reinterpret_cast<int8_t*>(base + qs),reinterpret_cast<float*>(base + d),mpad};
         PIX_HIP(pixhip::launch_quantize_q8_0(x,columns,K,kp,a,nullptr,s->stream),"quantize Q8_0");
-        e = pixhip::launch_gemm_q8_0(a,w->q80,columns,w->rows,K,out,nullptr,s->stream);
+        e = pixhip::gemm_q8_rows(columns,w->rows,K)? pixhip::launch_gemm_rows_q8_0(a,w->q80,columns,w->rows,K,out,s->stream)
+                                                   : pixhip::launch_gemm_q8_0(a,w->q80,columns,w->rows,K,out,nullptr,s->stream);
     } else {
         const size_t qs = c.take(mpad * K), d = c.take((K / PIX_QK) * mpad * 4), bs = c.take(mpad * (K / 16) * 2);
         if (c.offset > kNoAllocScratchBytes)

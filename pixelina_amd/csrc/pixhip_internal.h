@@ -254,6 +254,9 @@ hipError_t launch_gemm_q8_0(const Act80& a, const PlanarQ80& w, size_t M, size_t
 bool gemm_kq_rows(size_t M, size_t N, size_t K);
 hipError_t launch_gemm_rows_q5_K(const Act8K& a, const PlanesQ5K& w, size_t M, size_t N, size_t K, const Output& out, hipStream_t s);
 hipError_t launch_gemm_rows_q6_K(const Act8K& a, const PlanesQ6K& w, size_t M, size_t N, size_t K, const Output& out, hipStream_t s);
+// gemm_q8_rows.hip: the same for Q8_0.
+bool gemm_q8_rows(size_t M, size_t N, size_t K);
+hipError_t launch_gemm_rows_q8_0(const Act80& a, const PlanarQ80& w, size_t M, size_t N, size_t K, const Output& out, hipStream_t s);
 hipError_t launch_sums_q5_K(const Act8K& a, const PlanesQ5K& w, size_t M, size_t N, size_t K, int32_t* scaled, int32_t* mins,
                             hipStream_t s);
 hipError_t launch_sums_q6_K(const Act8K& a, const PlanesQ6K& w, size_t M, size_t N, size_t K, int32_t* sums, hipStream_t s);

@@ -214,3 +214,24 @@ def test_few_token_kquant(sess, wtype, m, n, k):
     x = rng.standard_normal((m, k)).astype(np.float32)
     ref = quant_matmul(oracle(), "orc", wb, wtype, x, n)
     assert row_rel_error(gpu_matmul(sess, wb, wtype, x, n), ref).max() <= 5e-6
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (2, 7, 32),          # one block, fewer features than a tile
+    (3, 97, 160),        # five blocks: the padded row ends inside a group of four
+    (31, 129, 1056),
+    (33, 4200, 224),     # two feature tiles a workgroup
+    (64, 5000, 96),
+    (100, 12300, 64),    # two tiles each way
+    (192, 600, 1248),
+    (700, 40, 2080),     # past the rows of one padded activation tile
+    (9, 1000, 4128),     # every wave has work
+])
+def test_few_token_q8_0(sess, m, n, k):
+    # exact integer block sums, fp32 sums over k / 32 <= 129 blocks in another order than the oracle's: 129 * 2^-24
+    # relative to the terms in the worst case
+    rng = np.random.default_rng(m * 31 + n)
+    wb = pack(Q8_0, (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    ref = quant_matmul(oracle(), "orc", wb, Q8_0, x, n)
+    assert row_rel_error(gpu_matmul(sess, wb, Q8_0, x, n), ref).max() <= 1e-5
