@@ -17,7 +17,7 @@
 // bits than an fp32 take fewer products: BF16 weights are one bf16 plane (two
 // products, the same sums), F16 weights one fp16 plane that multiplies an image
 // split in fp16 under a scale (two products; conv_body_ring).  256^2 pixels,
-// 512 -> 512, 3x3: three products 889 us, two fp16 721 (error against 64 bits
+// 512 -> 512, 3x3: three products 889 us, two fp16 706 (error against 64 bits
 // 3.8e-6 -> 6.2e-7), two bf16 678.
 //
 // Tile: 128 pixels x 128 output channels x 32 inner per stage, 4 waves of
@@ -135,13 +135,16 @@ __device__ __forceinline__ void half_planes(cu32x4 v, cu32x4& hi, cu32x4& lo)
     lo = cu32x4{b[0],b[1],b[2],b[3]};
 }
 
-// The fp16 split of a pair: hi truncated to fp16, lo = the remainders truncated
-// to fp16: 2^-20 of the value, or fp16's last place 2^-24 where that is more.
-__device__ __forceinline__ void halves2_f16(float a, float b, uint32_t& hi, uint32_t& lo)
+// The fp16 split of a pair times `scale` (a power of two): hi truncated to fp16,
+// lo = the remainders truncated to fp16: 2^-20 of the value, or fp16's last place
+// 2^-24 where that is more.  (The remainders as fused multiply-adds of the
+// unscaled values: the same exact differences, one mixed-precision instruction
+// each.)
+__device__ __forceinline__ void halves2_f16(float a, float b, float scale, uint32_t& hi, uint32_t& lo)
 {
-    const auto h = __builtin_amdgcn_cvt_pkrtz(a,b);
+    const auto h = __builtin_amdgcn_cvt_pkrtz(a * scale,b * scale);
     hi = __builtin_bit_cast(uint32_t,h);
-    lo = __builtin_bit_cast(uint32_t,__builtin_amdgcn_cvt_pkrtz(a - (float)h[0],b - (float)h[1]));
+    lo = __builtin_bit_cast(uint32_t,__builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(a,scale,-(float)h[0]),__builtin_fmaf(b,scale,-(float)h[1])));
 }
 
 __device__ __forceinline__ float weight_value(const uint8_t* raw, uint32_t type, size_t index)
@@ -470,7 +473,7 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
             ra[i] = make_float4(__uint_as_float(v.x),__uint_as_float(v.y),__uint_as_float(v.z),__uint_as_float(v.w));
         }
     };
-    float top[HALF? AV : 1];  // largest |x * scale| of this thread's share of each pixel's inputs
+    float top[HALF? AV : 1];  // largest |x| of this thread's share of each pixel's inputs
 #pragma unroll
     for (int i = 0; i < (HALF? AV : 1); i++) top[i] = 0.0f;
     auto store_a = [&](const float4 (&ra)[AV]) {
@@ -479,11 +482,10 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
             const int row = t / 8 + 32 * i, col = (t % 8) * 4;
             uint32_t h01, l01, h23, l23;
             if constexpr (HALF) {
-                const float x0 = ra[i].x * scale, x1 = ra[i].y * scale, x2 = ra[i].z * scale, x3 = ra[i].w * scale;
-                top[i] = __builtin_fmaxf(__builtin_fmaxf(top[i],__builtin_fabsf(x0)),__builtin_fabsf(x1));
-                top[i] = __builtin_fmaxf(__builtin_fmaxf(top[i],__builtin_fabsf(x2)),__builtin_fabsf(x3));
-                halves2_f16(x0,x1,h01,l01);
-                halves2_f16(x2,x3,h23,l23);
+                top[i] = __builtin_fmaxf(__builtin_fmaxf(top[i],__builtin_fabsf(ra[i].x)),__builtin_fabsf(ra[i].y));
+                top[i] = __builtin_fmaxf(__builtin_fmaxf(top[i],__builtin_fabsf(ra[i].z)),__builtin_fabsf(ra[i].w));
+                halves2_f16(ra[i].x,ra[i].y,scale,h01,l01);
+                halves2_f16(ra[i].z,ra[i].w,scale,h23,l23);
             } else {
                 halves2(ra[i].x,ra[i].y,h01,l01);
                 halves2(ra[i].z,ra[i].w,h23,l23);
@@ -604,7 +606,7 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
         bool outside = false;
 #pragma unroll
         for (int i = 0; i < AV; i++) {
-            float m = top[i];
+            float m = top[i] * scale;
             m = __builtin_fmaxf(m,dpp_f32<kDppXor1>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppXor2>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppHalfMirror>(m));
