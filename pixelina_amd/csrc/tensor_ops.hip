@@ -390,7 +390,9 @@ template <int VEC, bool KEEP> __device__ __forceinline__ typename Vec<VEC>::T gn
     }
 }
 
-template <int VEC>
+// KEEP: rows from keep_row on are read with plain loads (they stay in the
+// last-level cache for the apply pass).
+template <int VEC, bool KEEP>
 __global__ __launch_bounds__(256) void gn_partial_kernel(const float* __restrict__ x, GnShape sh, size_t keep_row, double* __restrict__ part)
 {
     typedef typename Vec<VEC>::T T;
@@ -414,9 +416,13 @@ __global__ __launch_bounds__(256) void gn_partial_kernel(const float* __restrict
     double sum[4] = {0.0,0.0,0.0,0.0};
     if (active) {
         // all loads first, then the sums (rows past the end add zero)
+        if (KEEP && row0 >= keep_row) {
 #pragma unroll
-        for (int k = 0; k < kGnRows; k++)
-            v[k] = row0 >= keep_row? gn_buffer_load<VEC,true>(rx,first + k * pitch) : gn_buffer_load<VEC,false>(rx,first + k * pitch);
+            for (int k = 0; k < kGnRows; k++) v[k] = gn_buffer_load<VEC,KEEP>(rx,first + k * pitch);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kGnRows; k++) v[k] = gn_buffer_load<VEC,false>(rx,first + k * pitch);
+        }
 #pragma unroll
         for (int k = 0; k < kGnRows; k++)
 #pragma unroll
@@ -547,10 +553,10 @@ __global__ __launch_bounds__(256) void gn_merge_kernel(const double* __restrict_
 }
 
 // With FIXED (256 a multiple of cvec) every value of a thread lies in one
-// column, whose weight, bias and group statistics are read once.  Spans run from
-// the last to the first: rows from keep_row on were left in the last-level cache
-// by the statistics pass.
-template <int VEC, bool FIXED, bool NT>
+// column, whose weight, bias and group statistics are read once.  With KEEP the
+// statistics pass left the rows from keep_row on in the last-level cache: the
+// spans run from the last to the first.
+template <int VEC, bool FIXED, bool NT, bool KEEP>
 __global__ __launch_bounds__(256) void gn_apply_kernel(const float* __restrict__ x, GnShape sh, const GnStat* __restrict__ stat,
                                                        const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y,
                                                        size_t keep_row)
@@ -574,9 +580,9 @@ __global__ __launch_bounds__(256) void gn_apply_kernel(const float* __restrict__
     }
     const size_t keep = keep_row * sh.cvec;
     for (size_t r = blockIdx.x; r < spans; r += gridDim.x) {
-        const size_t p = spans - 1 - r, base = p * span + threadIdx.x;
+        const size_t p = KEEP? spans - 1 - r : r, base = p * span + threadIdx.x;
         T v[kUnroll];
-        if (p * span >= keep) {
+        if (KEEP && p * span >= keep) {
 #pragma unroll
             for (int k = 0; k < kUnroll; k++)
                 if (base + k * (size_t)blockDim.x < total) v[k] = *reinterpret_cast<const T*>(x + (base + k * (size_t)blockDim.x) * VEC);
@@ -652,32 +658,38 @@ hipError_t launch_groupnorm(const float* x, const float* w, const float* b, floa
     const dim3 pgrid((unsigned)sh.chunks,(unsigned)sh.tiles), block(256);
     // The rows the apply pass finds in the last-level cache: it runs from the last
     // row down, and the statistics pass reads the last 224 MB with plain loads, the
-    // rows before them past the caches.  Us a call, everything past the caches /
-    // so: [1M, 128] 270 / 252, [256K, 512] 277 / 253, [1M, 96] 370 / 308.  Between
-    // 64 and 256 MB (plain output stores) wide rows lose, the output pushes the
-    // input out: [256K, 128] 82 / 90, [256K, 256] 147 / 158; rows below 512 bytes
-    // gain at every size ([340K, 96] 138 / 110, [500K, 64] 101 / 90).
+    // rows before them past the caches.  Us a call on three tensors in turn,
+    // everything past the caches and forwards / so: [100K, 96] (38 MB) 45.3 / 41.1,
+    // [100K, 128] 37.7 / 35.0, [600K, 128] (307 MB) 163.6 / 159.6, [1M, 128] 272.3
+    // / 268.9, [256K, 384] 211.6 / 206.2.  In between the output (plain stores)
+    // pushes the input out, and narrow rows lose: [500K, 64] 87.2 / 90.4, [1M, 64]
+    // 168 / 183, [256K, 256] (256 MB) 147 / 158.
     const size_t bytes = rows * channels * sizeof(float);
-    const bool keep = channels < 128 || bytes > kStreamBytes || bytes <= ((size_t)64 << 20);
+    const bool keep = bytes <= ((size_t)64 << 20) || (channels >= 128 && bytes > kStreamBytes);
     const size_t kept = keep? ((size_t)224 << 20) / (channels * sizeof(float)) : 0;
     const size_t keep_row = rows > kept? rows - kept : 0;
-    if (vec) gn_partial_kernel<4><<<pgrid,block,0,s>>>(x,sh,keep_row,part);
-    else gn_partial_kernel<1><<<pgrid,block,0,s>>>(x,sh,keep_row,part);
+    auto partial = [&](auto k) {
+        constexpr bool KEEP = decltype(k)::value;
+        if (vec) gn_partial_kernel<4,KEEP><<<pgrid,block,0,s>>>(x,sh,keep_row,part);
+        else gn_partial_kernel<1,KEEP><<<pgrid,block,0,s>>>(x,sh,keep_row,part);
+    };
+    if (keep) partial(std::true_type());
+    else partial(std::false_type());
     // at least 1024 chunks per first-level block
     const unsigned split = (unsigned)std::min<size_t>(kGnSplit,std::max<size_t>(1,(sh.chunks + 1023) / 1024));
     gn_merge_kernel<true><<<dim3(kGroups,split),block,0,s>>>(part,sh.chunks,sh,eps,level,stat);
     if (split > 1) gn_merge_kernel<false><<<dim3(kGroups,1),block,0,s>>>(level,split,sh,eps,nullptr,stat);
     const unsigned agrid = grid_unrolled(rows * sh.cvec);
     const bool fixed = 256 % sh.cvec == 0;
-    auto apply = [&](auto nt) {
-        constexpr bool NT = decltype(nt)::value;
-        if (vec && fixed) gn_apply_kernel<4,true,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
-        else if (vec) gn_apply_kernel<4,false,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
-        else if (fixed) gn_apply_kernel<1,true,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
-        else gn_apply_kernel<1,false,NT><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+    auto apply = [&](auto nt, auto k) {
+        constexpr bool NT = decltype(nt)::value, KEEP = decltype(k)::value;
+        if (vec && fixed) gn_apply_kernel<4,true,NT,KEEP><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+        else if (vec) gn_apply_kernel<4,false,NT,KEEP><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+        else if (fixed) gn_apply_kernel<1,true,NT,KEEP><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
+        else gn_apply_kernel<1,false,NT,KEEP><<<dim3(agrid),block,0,s>>>(x,sh,stat,w,b,y,keep_row);
     };
-    if (rows * channels * sizeof(float) > kStreamBytes) apply(std::true_type());
-    else apply(std::false_type());
+    if (bytes > kStreamBytes) keep? apply(std::true_type(),std::true_type()) : apply(std::true_type(),std::false_type());
+    else keep? apply(std::false_type(),std::true_type()) : apply(std::false_type(),std::false_type());
     return hipGetLastError();
 }
 
