@@ -480,8 +480,9 @@ typedef struct pixhip_conv_geometry {
  * tensor (F32 0, F16 1, BF16 30) of GGML shape [kernel_x, kernel_y,
  * in_channels, out_channels] (a rank-5 [kx, ky, 1, cin, cout] tensor is the
  * same bytes), keyed like pixhip_weight_get.  On first use it is made resident
- * as two bf16 planes (hi, lo = w - hi) with the inner index reordered to
- * (ky, kx, c); F16 and BF16 weights are exact in them.  Quantized convolution
+ * with the inner index reordered to (ky, kx, c): F32 weights as two bf16 planes
+ * (hi, lo = w - hi), BF16 as one bf16 plane, F16 as one fp16 plane (as two bf16
+ * planes, exactly, where in_channels is not a multiple of 32).  Quantized convolution
  * weights are PIXHIP_ERR_UNSUPPORTED. */
 int pixhip_conv_weight_get(pixhip_session* session, const char* key, const void* host_bytes, uint64_t bytes, uint32_t type,
                            uint64_t kernel_x, uint64_t kernel_y, uint64_t in_channels, uint64_t out_channels, pixhip_weight** out);
