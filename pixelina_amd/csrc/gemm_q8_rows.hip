@@ -88,7 +88,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_q8_rows_kernel(RowsArgs g)
         v4i a[kAhead][MT], w[kAhead][NT];
         float xd[kAhead][MT], wd[kAhead][NT];
         // Block u of chunk c into slot u.  A block past the last one repeats it
-        // (its weight scale is zeroed at use).
+        // (its scales are zeroed at use).
         auto load = [&](int c, int u) {
             const int b = min(c * kAhead + u,blocks - 1), at = (b >> 1) * 1024 + (b & 1) * 32;
 #pragma unroll
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_q8_rows_kernel(RowsArgs g)
                 const v16f fzero = {};
                 v4h xs[MT], ws[NT];
 #pragma unroll
-                for (int i = 0; i < MT; i++) xs[i] = scale_operand(xd[u][i]);
+                for (int i = 0; i < MT; i++) xs[i] = scale_operand(in? xd[u][i] : 0.0f);
 #pragma unroll
                 for (int j = 0; j < NT; j++) ws[j] = scale_operand(in? wd[u][j] : 0.0f);
                 __builtin_amdgcn_sched_barrier(0);
