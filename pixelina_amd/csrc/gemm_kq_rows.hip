@@ -319,7 +319,7 @@ bool gemm_kq_rows(size_t M, size_t N, size_t K)
     if (M <= 64) return true;
     double cost;
     choose_tile(M,N,&cost);
-    if (M > 128) return cost * (double)K <= 16.0 * 4096.0;
+    if (M > 128) return cost <= 16.0 && cost * (double)K <= 16.0 * 4096.0;
     if (cost > 28.0) return K >= 3072;
     if (K <= 8192 || N <= 8192) return true;
     int full, chunks;
