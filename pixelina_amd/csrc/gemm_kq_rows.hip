@@ -218,8 +218,8 @@ template <bool Q5, int MT, int NT> hipError_t launch_tile(RowsArgs g, hipStream_
 }
 
 // The tile of a call.  A workgroup's operand traffic per 64 values is 2*NT KB of
-// weights and MT KB of activations, and the busiest CU runs groups / CUs of
-// them (at least one): the tile with the least product of the two is taken.
+// weights and MT KB of activations, and the busiest XCD's CUs run groups / CUs
+// of them (at least one): the tile with the least product of the two is taken.
 // Measured, K = 4096, us a call: 48 tokens x 12288 features 3x1 26.7, 3x2 25.1;
 // 128 x 4096 4x1 21.3, 4x2 16.6, 8x1 19.7; 64 x 2048 (K = 12288) 2x1 20.6, 2x2
 // 25.7, 4x1 26.5.  Larger tiles (4x3, 6x2, 8x2) need more registers than two
@@ -238,8 +238,9 @@ Tile choose_tile(size_t M, size_t N, double* least_cost)
         const size_t rows = 16 * (size_t)t.mt;
         if (t.mt > 1 && rows - 16 >= M) continue;                // 16 rows of padding only
         if (PIX_GEMM_MTILE % rows && rows < M) continue;         // its last tile would leave the padding
-        const double groups = (double)((M + 16 * t.mt - 1) / (16 * t.mt)) * (double)((N + 16 * t.nt - 1) / (16 * t.nt));
-        const double cost = (2 * t.nt + t.mt) * std::max(1.0,groups / cus);
+        // workgroups of the busiest XCD (whole feature groups are dealt to the eight)
+        const double groups = (double)((M + rows - 1) / rows) * (double)((N + 128 * t.nt - 1) / (128 * t.nt));
+        const double cost = (2 * t.nt + t.mt) * std::max(1.0,groups / (cus / 8));
         if (least == 0.0 || cost < least) {
             least = cost;
             best = t;
@@ -310,16 +311,18 @@ hipError_t launch_gemm_rows_q6_K(const Act8K& a, const PlanesQ6K& w, size_t M, s
 //   M <= 128 (weights read by two token tiles): 58 / 44 (128 x 12288, K =
 //     4096), 29 / 16 (4096, 3584), but 24.2 / 29.5 (18944, 1024: cost 37) and
 //     101 / 105 (9728, 12288: its K pieces fill the device);
-//   above, only while the whole call is short: 29.4 / 26.0 (256 x 4096, K =
-//     3584), 31.0 / 21.6 (256 x 1000, 8192), but 42.1 / 49.2 (160 x 4096, 8192)
-//     and 31.9 / 34.8 (160 x 1000, 12288).
+//   above, only while the whole call is short: 23.5 / 21.3 (200 x 4000, K =
+//     2560), 31.0 / 21.6 (256 x 1000, 8192), 27.6 / 19.7 (900 x 500, 4096), 19.5 /
+//     15.7 (2000 x 500, 1024), but 27.5 / 33.3 (300 x 800, 8192), 42.1 / 49.2 (160 x 4096, 8192), 31.9 / 34.8
+//     (160 x 1000, 12288), 26.2 / 28.2 (2000 x 100, 4096) and 19.7 / 22.1 (4600 x
+//     100, 1024).
 bool gemm_kq_rows(size_t M, size_t N, size_t K)
 {
     if (K % PIX_QK) return false;
     if (M <= 64) return true;
     double cost;
     choose_tile(M,N,&cost);
-    if (M > 128) return cost <= 16.0 && cost * (double)K <= 16.0 * 4096.0;
+    if (M > 128) return M <= (K <= 1024? 2048u : 1024u) && cost <= 16.0 && cost * (double)K <= 16.0 * 3072.0;
     if (cost > 28.0) return K >= 3072;
     if (K <= 8192 || N <= 8192) return true;
     int full, chunks;

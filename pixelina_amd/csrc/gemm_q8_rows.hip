@@ -169,7 +169,7 @@ template <int MT, int NT> hipError_t launch_tile(RowsArgs g, hipStream_t s)
 // The tile of a call (us, one call, tiles 1x1 / 1x2 / 2x2 of 32: 37 x 12288 -> 4096
 // 29.4 / 41.1 / 58.0, 16 x 4096 -> 4096 11.5 / 14.5 / -, 128 x 4096 -> 12288 50.0 /
 // 43.1 / 43.3, 256 x 3840 -> 3840 28.8 / 25.3 / 20.6): a workgroup reads MT + NT KB per block of 32 values, and
-// the busiest CU runs groups / CUs of them (at least one); the least product of
+// the busiest XCD's CUs run groups / CUs of them (at least one); the least product of
 // the two is taken.
 int choose_tile(size_t M, size_t N, double* least_cost)
 {
@@ -179,8 +179,9 @@ int choose_tile(size_t M, size_t N, double* least_cost)
     for (const int t : {22,12,11}) {
         const size_t rows = 32 * (t / 10), features = 32 * (t % 10);
         if (rows > 32 && M <= 32) continue;
-        const double groups = (double)((M + rows - 1) / rows) * (double)((N + features - 1) / features);
-        const double cost = (t / 10 + t % 10) * std::max(1.0,groups / cus);
+        // workgroups of the busiest XCD (whole feature groups are dealt to the eight)
+        const double groups = (double)((M + rows - 1) / rows) * (double)((N + 8 * features - 1) / (8 * features));
+        const double cost = (t / 10 + t % 10) * std::max(1.0,groups / (cus / 8));
         if (least == 0.0 || cost < least) {
             least = cost;
             best = t;
@@ -226,7 +227,7 @@ bool gemm_q8_rows(size_t M, size_t N, size_t K)
 {
     double cost;
     choose_tile(M,N,&cost);
-    if (gemm_q8_0_grouped(M,N)) return cost <= 3.0 && (M <= 1024 || K <= 2048);
+    if (gemm_q8_0_grouped(M,N)) return cost <= 3.0 && M <= (K <= 2048? 2048u : 1024u);
     return M <= 192 && cost <= (K >= 1024? 9.5 : 9.0);
 }
 
