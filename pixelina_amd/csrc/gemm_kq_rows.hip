@@ -310,7 +310,8 @@ hipError_t launch_gemm_rows_q6_K(const Act8K& a, const PlanesQ6K& w, size_t M, s
 //     (33 x 18944, K = 12288), nowhere less than 1.2 times faster;
 //   M <= 128 (weights read by two token tiles): 58 / 44 (128 x 12288, K =
 //     4096), 29 / 16 (4096, 3584), but 24.2 / 29.5 (18944, 1024: cost 37) and
-//     101 / 105 (9728, 12288: its K pieces fill the device);
+//     101 / 105 (9728, 12288: its K pieces fill the device), 36 / 43 (70 x
+//     3000, 12288);
 //   above, only while the whole call is short: 23.5 / 21.3 (200 x 4000, K =
 //     2560), 31.0 / 21.6 (256 x 1000, 8192), 27.6 / 19.7 (900 x 500, 4096), 19.5 /
 //     15.7 (2000 x 500, 1024), but 27.5 / 33.3 (300 x 800, 8192), 42.1 / 49.2 (160 x 4096, 8192), 31.9 / 34.8
@@ -324,11 +325,11 @@ bool gemm_kq_rows(size_t M, size_t N, size_t K)
     choose_tile(M,N,&cost);
     if (M > 128) return M <= (K <= 1024? 2048u : 1024u) && cost <= 16.0 && cost * (double)K <= 16.0 * 3072.0;
     if (cost > 28.0) return K >= 3072;
-    if (K <= 8192 || N <= 8192) return true;
+    if (K <= 8192 || N <= 1024) return true;
     int full, chunks;
     const int splits = gemm_split_plan(M,N,K,full,chunks);
     const double groups = (double)full + ((double)((N + PIX_GEMM_NTILE - 1) / PIX_GEMM_NTILE) - full) * splits, cus = device_cus();
-    return groups < 0.85 * cus;
+    return groups < 0.8 * cus;
 }
 
 }  // namespace pixhip
