@@ -676,14 +676,17 @@ __global__ __launch_bounds__(256) void attn_combine(AttnArgs a)
         float mg = m;
 #pragma unroll
         for (int s = 0; s < 8; s++) mg = fmaxf(mg,ml[s].x);
-        const float old = __builtin_amdgcn_exp2f(m - mg);  // the first group: exp2(-inf) = 0
+        // (every piece so far may be empty: a causal unit of one key tile has
+        // its keys in the last piece)
+        const float mr = mg == -INFINITY? 0.0f : mg;
+        const float old = __builtin_amdgcn_exp2f(m - mr);  // the first group: exp2(-inf) = 0
         l *= old;
 #pragma unroll
         for (int i = 0; i < 4; i++) v[i] *= old;
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             // maxima in log2 units; an empty piece has -inf: weight 0
-            const float w = 8 * g + s < a.splits? __builtin_amdgcn_exp2f(ml[s].x - mg) : 0.0f;
+            const float w = 8 * g + s < a.splits? __builtin_amdgcn_exp2f(ml[s].x - mr) : 0.0f;
             l += w * ml[s].y;
             v[0] += w * x[s].x;
             v[1] += w * x[s].y;

@@ -149,6 +149,29 @@ def test_short_ranges_against_oracle(sess, rows, keys, heads, kvh, dim, causal, 
     assert np.array_equal(y.view(np.uint32), y2.view(np.uint32)), "repeats differ"
 
 
+@pytest.mark.parametrize("rows,keys,heads,kvh,dim", [
+    (520, 520, 2, 1, 128),   # packed heads: the first tile is 64 rows, one key tile of nine pieces
+    (640, 640, 4, 2, 64),    # ten pieces
+    (64, 1024, 8, 8, 128),   # sixteen pieces, all rows in one key tile
+    (33, 1024, 2, 2, 64),
+    (64, 600, 1, 1, 72),     # ten pieces of one unit
+])
+def test_causal_tiles_of_one_key_tile(sess, rows, keys, heads, kvh, dim):
+    """Causal rows from the first key on whose keys are cut into more than eight
+    pieces: a unit that sees one key tile leaves every piece but the last empty,
+    and the merge of the pieces starts with eight empty ones."""
+    rng = np.random.default_rng(rows * 31 + keys)
+    q, k, v = qkv(rng, rows, keys, heads, kvh, dim)
+    ranges = [(0, rows, keys, 1)]
+    print(f"rows={rows} keys={keys} heads={heads}/{kvh} dim={dim}", flush=True)
+    y = gpu_attention(sess, q, k, v, heads, kvh, ranges=ranges)
+    ref = attention(oracle(), "orc", q, k, v, heads, kvh, ranges)
+    assert np.isfinite(y).all(), f"{np.isnan(y).any(axis=1).sum()} rows are not finite"
+    err = row_rel_error(y, ref).max()
+    print(f"  rel={err:.2e}", flush=True)
+    assert err <= TOL
+
+
 def test_short_and_long_ranges_together(sess):
     """Ranges of one call on different kernels: 2 rows (few queries), 90 rows
     (tiled), 1 row limited to a key prefix."""
