@@ -606,11 +606,11 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
         bool outside = false;
 #pragma unroll
         for (int i = 0; i < AV; i++) {
-            float m = top[i] * scale;
+            float m = top[i];
             m = __builtin_fmaxf(m,dpp_f32<kDppXor1>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppXor2>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppHalfMirror>(m));
-            outside = outside || m > 32768.0f || (m != 0.0f && m < 0.015625f);
+            outside = outside || m * scale > 32768.0f || (m != 0.0f && m * scale < 0.015625f);
         }
         if (__syncthreads_or(outside)) return true;
         back = 1.0f / scale;
@@ -664,7 +664,7 @@ __device__ __forceinline__ float conv_scale(const ConvArgs& a, uint16_t* shared)
     most = __builtin_fmaxf(__builtin_fmaxf(waves[0],waves[1]),__builtin_fmaxf(waves[2],waves[3]));
     __syncthreads();
     const int e = (int)(__float_as_uint(most) >> 23);  // biased exponent: 2^(e - 127) <= most
-    const int s = e == 0 || e == 255? 130 : 130 - ((e - 124) >> 3) * 8;  // (10 .. 250)
+    const int s = e == 0 || e == 255? 130 : min(130 - ((e - 124) >> 3) * 8,250);  // (2 .. 250: a normal power of two)
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(s) << 23);
 }
 

@@ -128,6 +128,41 @@ def test_half_weights_over_the_range(sess, scale, geom):
     assert np.all(y[peak[:, 0] == 0] == 0)
 
 
+def conv64(x, width, height, w, k):
+    """The "same" convolution in 64 bits (odd k): w [cout][cin * k * k]."""
+    cin, cout = x.shape[1], w.shape[0]
+    img = np.pad(x.astype(np.float64).reshape(height, width, cin), ((k // 2, k // 2), (k // 2, k // 2), (0, 0)))
+    taps = w.astype(np.float64).reshape(cout, cin, k, k)
+    y = np.zeros((height, width, cout))
+    for dy in range(k):
+        for dx in range(k):
+            y += img[dy:dy + height, dx:dx + width] @ taps[:, :, dy, dx].T
+    return y.reshape(-1, cout)
+
+
+@pytest.mark.parametrize("low", ["1.5e-38", "5e-38", "9e-38", "2e-37", "1e37", "3e38"])
+@pytest.mark.parametrize("others", ["same", "channels", "pixels"])
+def test_half_weights_at_the_ends_of_the_exponent(sess, low, others):
+    """F16 weights and image values at either end of fp32's normal range: in all of
+    the image, in one channel beside ones and zeros, or in every other pixel
+    beside pixels at 1e-25.  The scale of a tile, taken from a sample of it,
+    stays a positive normal power of two, and nothing is lost to it."""
+    rng = np.random.default_rng(3)
+    wd, ht, cin, cout, k = 21, 13, 64, 40, 1
+    x = np.full((wd * ht, cin), np.float32(low), np.float32)
+    if others == "channels":
+        x[:, 1:] = 0
+        x[:, 32:36] = 1
+    elif others == "pixels":
+        x[1::2] = np.float32(1e-25)
+    w = (rng.standard_normal((cout, cin * k * k)) / 256).astype(np.float32)
+    raw, wv = weight_bytes(w, F16)
+    y = gpu_conv(sess, "conv:ends", x, wd, ht, raw, F16, k, k, cin, cout)
+    ref, top = conv64(x, wd, ht, wv, k), conv64(np.abs(x), wd, ht, np.abs(wv), k)
+    # sums of products below the smallest normal (2^-126) may lose bits, each at most 2^-133 (a bf16 half's last place)
+    assert np.all(np.abs(y - ref) <= 3 * 2.0 ** -17 * top + cin * 2.0 ** -133), float((np.abs(y - ref) / top).max())
+
+
 def test_vae_shape_band_and_translation(sess):
     """256 x 256 pixels, 512 -> 512 channels, 3x3 (a VAE decoder block's
     conv): output rows 0-1 and 127-128 against the oracle run on the input
