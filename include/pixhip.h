@@ -481,9 +481,9 @@ typedef struct pixhip_conv_geometry {
  * in_channels, out_channels] (a rank-5 [kx, ky, 1, cin, cout] tensor is the
  * same bytes), keyed like pixhip_weight_get.  On first use it is made resident
  * with the inner index reordered to (ky, kx, c): F32 weights as two bf16 planes
- * (hi, lo = w - hi), BF16 as one bf16 plane, F16 as one fp16 plane (as two bf16
- * planes, exactly, where in_channels is not a multiple of 32).  Quantized convolution
- * weights are PIXHIP_ERR_UNSUPPORTED. */
+ * (hi, lo = w - hi), BF16 as one bf16 plane, F16 as one fp16 plane and its rows'
+ * sums of magnitudes (as two bf16 planes, exactly, where in_channels is not a
+ * multiple of 32).  Quantized convolution weights are PIXHIP_ERR_UNSUPPORTED. */
 int pixhip_conv_weight_get(pixhip_session* session, const char* key, const void* host_bytes, uint64_t bytes, uint32_t type,
                            uint64_t kernel_x, uint64_t kernel_y, uint64_t in_channels, uint64_t out_channels, pixhip_weight** out);
 
@@ -494,8 +494,8 @@ int pixhip_conv_weight_get(pixhip_session* session, const char* key, const void*
  * `geometry` NULL is tensor_conv's first form (stride 1, the kernel centred at
  * offset kernel / 2, out = in); otherwise out_width = (width + left + right -
  * kernel_x) / stride_x + 1 (and likewise in y), with the reference's checks.
- * Within 1e-4 of the fp32 reference per output row (split-bf16 MFMA products,
- * fp32 accumulation).  Tensors are device or pinned host memory (input and
+ * Within 1e-4 of the fp32 reference per output row (split products on MFMA,
+ * fp32 accumulation): each output within 2^-15 of its own sum |x| |w|.  Tensors are device or pinned host memory (input and
  * bias may be pageable), 4-byte aligned.  Images of more than 2^32 - 1 pixels
  * are PIXHIP_ERR_ARGUMENT. */
 int pixhip_conv2d(pixhip_session* session, const pixhip_weight* weight, const float* input, size_t width, size_t height,

@@ -73,10 +73,12 @@ def _compile(src):
 # the counter completely and are exempt).  The attention kernels drain it
 # completely too, but sit at the register limit, where a spill would mean
 # scratch traffic in the key loop; they are checked as well, as are the few-token
-# kernels (a tile that spilled ran three times slower).
+# kernels (a tile that spilled ran three times slower) and the convolution's
+# (its 16-bit forms, 15% and more slower with a spill in the loop).
 NO_SPILL = {
     "csrc/attention.hip": ("attn_kernelILi128ELi1E", "attn_kernelILi128ELi2E", "attn_kernelILi64ELi1E", "attn_kernelILi64ELi2E", "attn_wide_kernelILi128E", "attn_wide_kernelILi96E",
                            "attn_wide_kernelILi64E"),
+    "csrc/conv.hip": ("conv_image_kernelILi1E", "conv_image_kernelILi2E"),
     "csrc/gemm_kq.hip": ("gemm_kq_kernelILb1ELb0E", "gemm_kq_kernelILb0ELb0E"),
     "csrc/gemm_kq_rows.hip": ("gemm_kq_rows_kernel",),
     "csrc/gemm_q8_rows.hip": ("gemm_q8_rows_kernel",),

@@ -1864,10 +1864,12 @@ int ensure_conv_form(pixhip_session* s, pixhip_weight* w)
     if (rc) return rc;
     const size_t plane = w->conv_npad * w->conv_kp * sizeof(uint16_t);
     const int kind = pixhip::conv_weight_kind(w->type,(int)w->cin);
-    if ((rc = weight_alloc(s,w,(kind == pixhip::kConvSplit? 2 : 1) * plane,&w->conv_planes))) return rc;
-    uint16_t* hi = static_cast<uint16_t*>(w->conv_planes);
+    // (the fp16 plane is followed by its rows' sums of magnitudes)
+    const size_t bytes = kind == pixhip::kConvSplit? 2 * plane : kind == pixhip::kConvHalf? plane + w->conv_npad * sizeof(float) : plane;
+    if ((rc = weight_alloc(s,w,bytes,&w->conv_planes))) return rc;
+    uint16_t *hi = static_cast<uint16_t*>(w->conv_planes), *next = hi + plane / sizeof(uint16_t);
     PIX_HIP(pixhip::launch_conv_form(w->raw,w->type,(int)w->kernel_x,(int)w->kernel_y,(int)w->cin,(int)w->rows,(int)w->conv_kp,
-                                     (int)w->conv_npad,kind,hi,hi + plane / sizeof(uint16_t),s->stream),
+                                     (int)w->conv_npad,kind,hi,next,reinterpret_cast<float*>(next),s->stream),
             "convolution weight form");
     return release_raw(s,w);
 }
@@ -1976,7 +1978,9 @@ int pixhip_conv2d(pixhip_session* s, const pixhip_weight* wc, const float* input
     a.x = static_cast<const float*>(in);
     a.wh = static_cast<const uint16_t*>(w->conv_planes);
     a.kind = pixhip::conv_weight_kind(w->type,(int)w->cin);
-    a.wl = a.kind == pixhip::kConvSplit? a.wh + w->conv_npad * w->conv_kp : nullptr;
+    const uint16_t* const next = a.wh + w->conv_npad * w->conv_kp;
+    if (a.kind == pixhip::kConvSplit) a.wl = next;
+    if (a.kind == pixhip::kConvHalf) a.wsum = reinterpret_cast<const float*>(next);
     a.bias = static_cast<const float*>(b);
     a.y = static_cast<float*>(out);
     a.W = (int)width;

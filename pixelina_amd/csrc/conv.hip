@@ -17,8 +17,8 @@
 // bits than an fp32 take fewer products: BF16 weights are one bf16 plane (two
 // products, the same sums), F16 weights one fp16 plane that multiplies an image
 // split in fp16 under a scale (two products; conv_body_ring).  256^2 pixels,
-// 512 -> 512, 3x3: three products 889 us, two fp16 706 (error against 64 bits
-// 3.8e-6 -> 6.2e-7), two bf16 678.
+// 512 -> 512, 3x3: three products 881 us, two fp16 708 (error against 64 bits
+// 4.5e-6 / 6.2e-7), two bf16 665.
 //
 // Tile: 128 pixels x 128 output channels x 32 inner per stage, 4 waves of
 // 64 x 64 (2 x 2 MFMA tiles).  The image kernel (images below 2 GiB) keeps one
@@ -195,12 +195,26 @@ __global__ __launch_bounds__(256) void conv_form_kernel(const uint8_t* __restric
     }
 }
 
+// sums[n] = sum of |w| over row n of an fp16 plane, one wave per row.
+__global__ __launch_bounds__(64) void conv_row_sums_kernel(const uint16_t* __restrict__ plane, int kp, float* __restrict__ sums)
+{
+    float v = 0.0f;
+    for (int k = 8 * (int)threadIdx.x; k < kp; k += 512) {
+        const v8h h = *reinterpret_cast<const v8h*>(plane + (size_t)blockIdx.x * kp + k);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v += __builtin_fabsf((float)h[i]);
+    }
+    v = wave_sum(v);
+    if (threadIdx.x == 0) sums[blockIdx.x] = v;
+}
+
 hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad, int kind,
-                            uint16_t* hi, uint16_t* lo, hipStream_t s)
+                            uint16_t* hi, uint16_t* lo, float* sums, hipStream_t s)
 {
     const size_t total = (size_t)npad * kp;
     const unsigned grid = (unsigned)std::min<size_t>((total + 255) / 256,(size_t)1 << 20);
     conv_form_kernel<<<dim3(grid),dim3(256),0,s>>>(static_cast<const uint8_t*>(raw),type,kernel_x,kernel_y,cin,cout,kp,npad,kind,hi,lo);
+    if (kind == kConvHalf) conv_row_sums_kernel<<<dim3((unsigned)npad),dim3(64),0,s>>>(hi,kp,sums);
     return hipGetLastError();
 }
 
@@ -376,6 +390,146 @@ __device__ __forceinline__ void conv_body(const ConvArgs& a)
 }
 
 
+// How a tile of the fp16 form is held, from a sample of its inner range: the
+// centre tap's first 32 channels and, where an output is not held by those, the
+// first 32 of the other taps in turn.
+//   scale  a power of two from the largest |x| at the centre tap, in steps of
+//          2^2: 2^7 for 2 .. 8, so that neighbouring tiles, and the same values
+//          at another place of another image, mostly split alike.  The largest
+//          becomes 2^8 .. 2^10: 64 times as much still fits fp16, and a pixel of
+//          normal values may be 50 times dimmer than the tile's brightest (at
+//          4608 inner values) before it is not held.  0 where an output whose
+//          pixel is not blank is not held: its share of the sum |x| |w| in the
+//          sample is less than kLeast of its sum |w|;
+//   blank  bit i: the sample holds only zeros for this thread's pixel t / 8 + 32 i.
+// With FURTHER false only the centre tap is looked at, and scale is 0 unless it
+// holds every output (all but a few tiles): a stage without its pipelining, and
+// half of its products.
+constexpr float kLeast = 1.01f / 128;  // 2^-7, and 1% for the sum's rounding
+struct ConvProbe {
+    float scale;
+    int blank;
+};
+template <bool FURTHER>
+__device__ __forceinline__ ConvProbe conv_probe(const ConvArgs& a, uint16_t* lds, uint16_t* bs)
+{
+    // (opaque: values shared with the loop would sit in registers through it)
+    int t = threadIdx.x;
+    uint32_t tile_m = blockIdx.x, tile_n = blockIdx.y;
+    __asm__ volatile("" : "+v"(t), "+s"(tile_m), "+s"(tile_n));
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), lr = lane & 31, hh = lane >> 5;
+    const int wm = wave & 1, wn = wave >> 1;
+    const long long m0 = (long long)tile_m * 128;
+    const int n0 = (int)tile_n * kCN, taps = FURTHER? a.KX * a.KY : 1, centre = a.KY / 2 * a.KX + a.KX / 2;
+    float* const waves = reinterpret_cast<float*>(lds + 128 * kCRow);  // [4]
+    float* const most = waves + 4;                                     // [128]: the pixels' maxima (FURTHER)
+    ConvProbe probe = {0.0f,0};
+    float row[4] = {0.0f,0.0f,0.0f,0.0f};
+    v16f sum[2][2] = {};
+    bool held = true, lost = false;
+    for (int p = 0; p < taps; p++) {
+        const int tap = p == 0? centre : p <= centre? p - 1 : p;
+        const int ky = tap / a.KX, kx = tap % a.KX;
+        cu32x4 rb[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int q = t + 256 * j;
+            rb[j] = *reinterpret_cast<const cu32x4*>(a.wh + (size_t)(n0 + q / 4) * a.Kp + (size_t)tap * a.C + 8 * (q % 4));
+        }
+        float4 ra[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t m = (uint32_t)m0 + t / 8 + 32 * i, oy = m / (uint32_t)a.OW, ox = m - oy * (uint32_t)a.OW;
+            const int iy = (int)oy * a.SY - a.PT + ky, ix = (int)ox * a.SX - a.PL + kx;
+            ra[i] = make_float4(0.0f,0.0f,0.0f,0.0f);
+            if (m < a.M && iy >= 0 && iy < a.H && ix >= 0 && ix < a.W)
+                ra[i] = *reinterpret_cast<const float4*>(a.x + ((size_t)iy * a.W + ix) * a.C + (t % 8) * 4);
+            float v = __builtin_fmaxf(__builtin_fabsf(ra[i].x),__builtin_fabsf(ra[i].y));
+            v = __builtin_fmaxf(__builtin_fmaxf(v,__builtin_fabsf(ra[i].z)),__builtin_fabsf(ra[i].w));
+            v = __builtin_fmaxf(v,dpp_f32<kDppXor1>(v));
+            v = __builtin_fmaxf(v,dpp_f32<kDppXor2>(v));
+            row[i] = __builtin_fmaxf(row[i],__builtin_fmaxf(v,dpp_f32<kDppHalfMirror>(v)));
+        }
+        if (p == 0) {
+            float v = __builtin_fmaxf(__builtin_fmaxf(row[0],row[1]),__builtin_fmaxf(row[2],row[3]));
+            v = __builtin_fmaxf(v,dpp_f32<kDppMirror>(v));
+            v = __builtin_fmaxf(__builtin_fmaxf(lane_f32(v,0),lane_f32(v,16)),__builtin_fmaxf(lane_f32(v,32),lane_f32(v,48)));
+            if (lane == 0) waves[wave] = v;
+            __syncthreads();
+            v = __builtin_fmaxf(__builtin_fmaxf(waves[0],waves[1]),__builtin_fmaxf(waves[2],waves[3]));
+            const int e = (int)(__float_as_uint(v) >> 23);  // biased exponent: 2^(e - 127) <= v
+            const int s = e == 0 || e == 255? 134 : min(134 - ((e - 128) >> 1) * 2,250);  // (8 .. 250: a normal power of two)
+            probe.scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(s) << 23);
+        }
+        // |x| * scale (its fp16 hi, not above it) and |w| into LDS, as the ring
+        // has them; rows past the image hold fp16's largest
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = t / 8 + 32 * i;
+            const bool past = m0 + r >= a.M;
+            uint32_t h01, h23, l;
+            halves2_f16(__builtin_fabsf(ra[i].x),__builtin_fabsf(ra[i].y),probe.scale,h01,l);
+            halves2_f16(__builtin_fabsf(ra[i].z),__builtin_fabsf(ra[i].w),probe.scale,h23,l);
+            *reinterpret_cast<uint2*>(lds + r * kCRow + (t % 8) * 4) = past? make_uint2(0x7BFF7BFFu,0x7BFF7BFFu) : make_uint2(h01,h23);
+            if (FURTHER && t % 8 == 0) most[r] = past? -1.0f : row[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int q = t + 256 * j, r = q / 4;
+            *reinterpret_cast<cu32x4*>(bs + r * 32 + (((q % 4) ^ ((r >> 2) & 3)) << 3)) = rb[j] & 0x7FFF7FFFu;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            v8h x[2], w[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int r = wn * 64 + j * 32 + lr;
+                x[j] = *reinterpret_cast<const v8h*>(lds + (wm * 64 + j * 32 + lr) * kCRow + ks * 16 + 8 * hh);
+                w[j] = *reinterpret_cast<const v8h*>(bs + r * 32 + (((2 * ks + hh) ^ ((r >> 2) & 3)) << 3));
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i],w[j],sum[i][j],0,0,0);
+        }
+        held = true;
+        float far = 0.0f;  // the largest |x| of a pixel with an output that is not held
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float least = a.wsum[n0 + wn * 64 + 32 * j + lr] * kLeast;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if constexpr (FURTHER) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const float m = most[wm * 64 + 32 * i + 8 * (r / 4) + 4 * hh + r % 4];
+                        const bool in = (sum[i][j][r] >= least) | (m < 0.0f);
+                        held = held & in;
+                        far = __builtin_fmaxf(far,in? 0.0f : m);
+                    }
+                } else {
+                    float v = sum[i][j][0];
+#pragma unroll
+                    for (int r = 1; r < 16; r++) v = __builtin_fminf(v,sum[i][j][r]);
+                    held = held & (v >= least);
+                }
+            }
+        }
+        lost = far != 0.0f;
+        held = __syncthreads_and(held);
+        if (held) break;
+    }
+    if constexpr (FURTHER) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) probe.blank |= row[i] == 0.0f? 1 << i : 0;
+        if (__syncthreads_or(lost)) probe.scale = 0.0f;
+    } else if (!held) {
+        probe.scale = 0.0f;
+    }
+    return probe;
+}
+
 // The image kernel for images below 2 GiB, pipelined deeper than conv_body:
 // the weight planes go L2 -> LDS by buffer_load ... lds into a two-slot ring
 // (64-byte rows, piece c of row r at c ^ ((r >> 2) & 3), no registers), and
@@ -388,18 +542,26 @@ __device__ __forceinline__ void conv_body(const ConvArgs& a)
 //   kConvSplit  three bf16 products of split weights and image;
 //   kConvBf16   the weight is one bf16 plane: two products, the same sums;
 //   kConvHalf   the weight is one fp16 plane: two fp16 products of the image
-//               times `scale` (a power of two), split as hi + lo in fp16.
-//               Returns true, without an output, where an output pixel's
-//               inputs leave the range in which that split is at least as fine
-//               as the bf16 one: their largest |x * scale| above 2^15, or
-//               below 2^-6 and not zero (fp16's last place, 2^-24, is then
-//               more than 2^-18 of it);
-//   kConvWiden  the second try of those tiles: the plane widened to bf16
-//               halves, three bf16 products, one stage at a time.
+//               times `scale` (a power of two), split as hi + lo in fp16, for
+//               tiles that can be held this way (conv_probe);
+//   kConvWiden  the others: the plane widened to bf16 halves, three bf16
+//               products, one stage at a time.
+//
+// The fp16 split leaves an output an error of at most 2^-20 of its sum |x| |w|
+// plus 2^-24 / scale (fp16's last place) of its sum |w|.  The second term must
+// stay below 2^-17 of the sum |x| |w| (three bf16 products leave up to 2^-15),
+// whatever the magnitudes of the channels and weights are: the sum of the scaled
+// image must be kLeast of the sum |w| or more, which conv_probe shows with a
+// sample's share of it.  Where a pixel that the sample holds only zeros of has
+// other values, or a scaled value leaves fp16's range, kConvHalf returns true,
+// without an output.  256^2 pixels, 512 -> 512, 3x3, us: 708 (700 without the
+// bound, three products 881); with half of the pixels 2^12 times dimmer, every
+// tile on its second try, 954; a border of zeros, whose tiles take the longer
+// look, 788 (64^2 pixels: 70, three products 75, with the border 105).
 constexpr int kConvWiden = 3;
-template <int FORM>
-__device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, uint16_t (&lds)[2 * 128 * kCRow],
-                                               uint16_t (&bslot0)[2 * kCN * 32], uint16_t (&bslot1)[2 * kCN * 32])
+template <int FORM, int B0, int B1>
+__device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, const ConvProbe& probe, uint16_t (&lds)[2 * 128 * kCRow],
+                                               uint16_t (&bslot0)[B0], uint16_t (&bslot1)[B1])
 {
     constexpr bool WIDEN = FORM == kConvWiden, SPLIT = FORM == kConvSplit || WIDEN, HALF = FORM == kConvHalf;
     constexpr int CHUNKS = SPLIT? 4 : 2;  // weight transfers of a wave per stage
@@ -420,9 +582,9 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
     for (int i = 0; i < AV; i++) {
         const long long m = m0 + t / 8 + 32 * i;
         if (m < a.M) {
-            const int oy = (int)(m / a.OW), ox = (int)(m % a.OW);
-            iy0[i] = oy * a.SY - a.PT;
-            ix0[i] = ox * a.SX - a.PL;
+            const uint32_t oy = (uint32_t)m / (uint32_t)a.OW, ox = (uint32_t)m - oy * (uint32_t)a.OW;
+            iy0[i] = (int)oy * a.SY - a.PT;
+            ix0[i] = (int)ox * a.SX - a.PL;
         } else {
             iy0[i] = -(1 << 30);
             ix0[i] = 0;
@@ -476,6 +638,7 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
     float top[HALF? AV : 1];  // largest |x| of this thread's share of each pixel's inputs
 #pragma unroll
     for (int i = 0; i < (HALF? AV : 1); i++) top[i] = 0.0f;
+    const float scale = probe.scale;
     auto store_a = [&](const float4 (&ra)[AV]) {
 #pragma unroll
         for (int i = 0; i < AV; i++) {
@@ -610,7 +773,7 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
             m = __builtin_fmaxf(m,dpp_f32<kDppXor1>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppXor2>(m));
             m = __builtin_fmaxf(m,dpp_f32<kDppHalfMirror>(m));
-            outside = outside || m * scale > 32768.0f || (m != 0.0f && m * scale < 0.015625f);
+            outside = outside || m * scale > 65504.0f || (m != 0.0f && (probe.blank >> i & 1));
         }
         if (__syncthreads_or(outside)) return true;
         back = 1.0f / scale;
@@ -632,40 +795,25 @@ __device__ __forceinline__ bool conv_body_ring(const ConvArgs& a, float scale, u
     return false;
 }
 
-// The scale of an fp16 tile, a power of two from the largest |x| of a sample
-// (the centre tap's first 32 channels of the tile's pixels), in steps of 2^8:
-// 8 for a sample in 1/8 .. 32, so that neighbouring tiles, and the same values
-// at another place of another image, split alike.  The scaled sample is 1 ..
-// 256: the split is then fine for values up to 2^7 times the sample and for
-// pixels down to 2^-6 of it.
-__device__ __forceinline__ float conv_scale(const ConvArgs& a, uint16_t* shared)
+// The longer look and the second try are calls: inlined, their values take
+// registers from the first try's loop.
+typedef __attribute__((address_space(3))) uint8_t SharedBytes;
+typedef const __attribute__((address_space(4))) ConvArgs KernelArgs;
+__device__ __forceinline__ const ConvArgs& kernel_args(KernelArgs* args)
 {
-    const int t = threadIdx.x;
-    const long long m0 = (long long)blockIdx.x * 128;
-    float most = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const long long m = m0 + t / 8 + 32 * i;
-        const int iy = (int)(m / a.OW) * a.SY - a.PT + a.KY / 2, ix = (int)(m % a.OW) * a.SX - a.PL + a.KX / 2;
-        if (m < a.M && iy >= 0 && iy < a.H && ix >= 0 && ix < a.W) {
-            const float4 v = *reinterpret_cast<const float4*>(a.x + ((size_t)iy * a.W + ix) * a.C + (t % 8) * 4);
-            most = __builtin_fmaxf(__builtin_fmaxf(most,__builtin_fabsf(v.x)),__builtin_fabsf(v.y));
-            most = __builtin_fmaxf(__builtin_fmaxf(most,__builtin_fabsf(v.z)),__builtin_fabsf(v.w));
-        }
-    }
-    most = __builtin_fmaxf(most,dpp_f32<kDppXor1>(most));
-    most = __builtin_fmaxf(most,dpp_f32<kDppXor2>(most));
-    most = __builtin_fmaxf(most,dpp_f32<kDppHalfMirror>(most));
-    most = __builtin_fmaxf(most,dpp_f32<kDppMirror>(most));
-    most = __builtin_fmaxf(__builtin_fmaxf(lane_f32(most,0),lane_f32(most,16)),__builtin_fmaxf(lane_f32(most,32),lane_f32(most,48)));
-    float* waves = reinterpret_cast<float*>(shared);
-    if ((t & 63) == 0) waves[t >> 6] = most;
-    __syncthreads();
-    most = __builtin_fmaxf(__builtin_fmaxf(waves[0],waves[1]),__builtin_fmaxf(waves[2],waves[3]));
-    __syncthreads();
-    const int e = (int)(__float_as_uint(most) >> 23);  // biased exponent: 2^(e - 127) <= most
-    const int s = e == 0 || e == 255? 130 : min(130 - ((e - 124) >> 3) * 8,250);  // (2 .. 250: a normal power of two)
-    return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(s) << 23);
+    const uint64_t p = (uint64_t)args;  // (the same in every lane)
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32));
+    return *(const ConvArgs*)(KernelArgs*)(lo | hi << 32);
+}
+__device__ __attribute__((noinline)) ConvProbe conv_longer_look(KernelArgs* args, SharedBytes* lds, SharedBytes* bslot0)
+{
+    return conv_probe<true>(kernel_args(args),(uint16_t*)(uint8_t*)lds,(uint16_t*)(uint8_t*)bslot0);
+}
+__device__ __attribute__((noinline)) void conv_second_try(KernelArgs* args, SharedBytes* lds, SharedBytes* bslot0, SharedBytes* bslot1)
+{
+    const ConvProbe probe = {1.0f,0};
+    conv_body_ring<kConvWiden>(kernel_args(args),probe,*(uint16_t(*)[2 * 128 * kCRow])(uint8_t*)lds,
+                               *(uint16_t(*)[2 * kCN * 32])(uint8_t*)bslot0,*(uint16_t(*)[kCN * 32])(uint8_t*)bslot1);
 }
 
 template <int FORM>
@@ -673,13 +821,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3,3))) void
 {
     // (separate arrays: the compiler can then tell the image stores from the
     // transfers in flight into the ring)
+    constexpr bool HALF = FORM == kConvHalf;
     __shared__ __attribute__((aligned(1024))) uint16_t lds[2 * 128 * kCRow];
     __shared__ __attribute__((aligned(1024))) uint16_t bslot0[2 * kCN * 32];  // ring slots: planes hi, lo
-    __shared__ __attribute__((aligned(1024))) uint16_t bslot1[2 * kCN * 32];
-    if constexpr (FORM == kConvHalf) {
-        if (conv_body_ring<kConvHalf>(a,conv_scale(a,lds),lds,bslot0,bslot1)) conv_body_ring<kConvWiden>(a,1.0f,lds,bslot0,bslot1);
+    __shared__ __attribute__((aligned(1024))) uint16_t bslot1[(FORM == kConvSplit? 2 : 1) * kCN * 32];
+    ConvProbe probe = {1.0f,0};
+    if constexpr (HALF) {
+        auto args = (KernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+        auto *l = (SharedBytes*)(uint8_t*)lds, *b0 = (SharedBytes*)(uint8_t*)bslot0;
+        probe = conv_probe<false>(a,lds,bslot0);
+        if (probe.scale == 0.0f) {
+            probe = conv_longer_look(args,l,b0);
+            probe.scale = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(probe.scale)));
+        }
+        if (probe.scale == 0.0f || conv_body_ring<kConvHalf>(a,probe,lds,bslot0,bslot1))
+            conv_second_try(args,l,b0,(SharedBytes*)(uint8_t*)bslot1);
     } else {
-        conv_body_ring<FORM>(a,1.0f,lds,bslot0,bslot1);
+        conv_body_ring<FORM>(a,probe,lds,bslot0,bslot1);
     }
 }
 
@@ -704,12 +862,13 @@ __global__ __launch_bounds__(256) void conv_reduce_kernel(const float* __restric
     y[e] = bias? __fadd_rn(v,bias[e % (unsigned)N]) : v;
 }
 
-// Whether a call runs the image kernel (a stage is whole channels, 32-bit offsets).
+// Whether a call runs the image kernel (a stage is whole channels, 32-bit offsets
+// and pixels).
 static bool image_form(const ConvArgs& a)
 {
     const size_t lim = (size_t)1 << 31;
     return a.C % kCK == 0 && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && (size_t)a.W * a.H * a.C * 4 < lim &&
-           (size_t)a.Npad * a.Kp * 2 < lim;
+           (size_t)a.Npad * a.Kp * 2 < lim && a.M < (long long)lim;
 }
 
 // Pieces of the inner range for images whose tiles leave CUs idle (one: none).

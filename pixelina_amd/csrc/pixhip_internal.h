@@ -206,12 +206,13 @@ struct ConvArgs {
     int W, H, C, KX, KY, SX, SY, PL, PT, OW, OH, K, Kp, N, Npad;
     long long M;
     int kind;  // the weight's form; wl is read for kConvSplit only
+    const float* wsum;  // kConvHalf: the sum of |w| of each of the Npad rows
     float* part;       // pieces of the inner range: their sums [piece][M][N] (launch_conv sets both)
     int piece_stages;
 };
 constexpr int kConvTileN = 128, kConvTileK = 32;
 hipError_t launch_conv_form(const void* raw, uint32_t type, int kernel_x, int kernel_y, int cin, int cout, int kp, int npad, int kind,
-                            uint16_t* hi, uint16_t* lo, hipStream_t s);
+                            uint16_t* hi, uint16_t* lo, float* sums, hipStream_t s);
 // Pieces of the inner range a call is worth cutting into (1: none); launch_conv
 // takes a workspace of pieces * M * N floats for them, or null to run whole.
 int conv_pieces(const ConvArgs& a);

@@ -128,6 +128,12 @@ def test_half_weights_over_the_range(sess, scale, geom):
     assert np.all(y[peak[:, 0] == 0] == 0)
 
 
+# Of an output's sum |x| |w|, what three products of bf16 halves may leave: the
+# image's low half is within 2^-8 of 2^-8 of the value, the dropped product of the
+# low halves is 2^-8 of 2^-8 of the term (fp32 sums add less than 1% to that here).
+THREE_PRODUCTS = 2.0 ** -15
+
+
 def conv64(x, width, height, w, k):
     """The "same" convolution in 64 bits (odd k): w [cout][cin * k * k]."""
     cin, cout = x.shape[1], w.shape[0]
@@ -160,7 +166,74 @@ def test_half_weights_at_the_ends_of_the_exponent(sess, low, others):
     y = gpu_conv(sess, "conv:ends", x, wd, ht, raw, F16, k, k, cin, cout)
     ref, top = conv64(x, wd, ht, wv, k), conv64(np.abs(x), wd, ht, np.abs(wv), k)
     # sums of products below the smallest normal (2^-126) may lose bits, each at most 2^-133 (a bf16 half's last place)
-    assert np.all(np.abs(y - ref) <= 3 * 2.0 ** -17 * top + cin * 2.0 ** -133), float((np.abs(y - ref) / top).max())
+    assert np.all(np.abs(y - ref) <= THREE_PRODUCTS * top + cin * 2.0 ** -133), float((np.abs(y - ref) / top).max())
+
+
+@pytest.mark.parametrize("spread", [64, 1024, 1e6, 1e9, 1e12])
+@pytest.mark.parametrize("dim", [1, 2.0 ** -7, 2.0 ** -12])
+@pytest.mark.parametrize("k", [1, 3])
+def test_half_weights_keep_every_channel(sess, spread, dim, k):
+    """F16 weights and channels of very different magnitudes within each pixel
+    (down to 1 / spread of the largest), half of the pixels `dim` times as bright:
+    outputs that read one class of channels only, and outputs whose weights are
+    the larger the smaller the channel (as far as F16 goes).  Each output is held
+    to the three bf16 products' bound of its OWN terms."""
+    rng = np.random.default_rng(int(spread) % 1000 + k)
+    wd, ht, cin, cout = 37, 21, 64, 72
+    size = spread ** -rng.random(cin)
+    size[:4], size[32:36] = 1, 1 / spread
+    x = rng.standard_normal((wd * ht, cin)) * size
+    x[rng.random(wd * ht) < 0.5] *= dim
+    x = x.astype(np.float32)
+    w = rng.standard_normal((cout, cin, k * k)) / 64
+    for n in range(0, 48):
+        w[n, np.abs(np.log(size) - np.log(rng.choice(size))) > 0.5] = 0  # one class of channels
+    w[48:60] *= np.minimum(1 / size, 1e4)[None, :, None] / 16
+    raw, wv = weight_bytes(np.ascontiguousarray(w.reshape(cout, -1), np.float32), F16)
+    y = gpu_conv(sess, f"conv:channels:{spread}:{dim}:{k}", x, wd, ht, raw, F16, k, k, cin, cout)
+    ref, top = conv64(x, wd, ht, wv, k), conv64(np.abs(x), wd, ht, np.abs(wv), k)
+    err = np.abs(y - ref) / np.maximum(top, 1e-37)
+    print(f"spread {spread} dim {dim} k {k}: worst {err.max():.2e} of an output's own terms", flush=True)
+    assert err.max() <= THREE_PRODUCTS
+
+
+@pytest.mark.parametrize("case", ["empty sample", "empty centre", "empty border", "beyond fp16", "one channel", "not a number"])
+def test_half_weights_beyond_the_sample(sess, case):
+    """F16 weights where the sample that an fp16 tile is judged by (the first 32
+    channels, the centre tap before the others) says little of the rest: zeros in
+    it, in all pixels or in some, values far larger than any of it, weights that
+    read one channel of it, NaN and Inf past it.  Held to the same bound of each
+    output's own terms; NaN and Inf reach the outputs they reach in fp32."""
+    rng = np.random.default_rng(11)
+    wd, ht, cin, cout, k = 37, 21, 96, 72, 3
+    x = rng.standard_normal((ht, wd, cin)).astype(np.float32)
+    w = rng.standard_normal((cout, cin, k * k)) / 32
+    if case == "empty sample":
+        x[:, :, :32] = 0
+    elif case == "empty centre":
+        x[::2, ::2] = 0
+        x[8:14, :, :64] = 0
+    elif case == "empty border":
+        x[:, :3] = 0
+        x[-4:] = 0
+    elif case == "beyond fp16":
+        x[10:, 20:, 40] *= 1e6
+    elif case == "one channel":
+        w[:36] = 0
+        w[np.arange(36), rng.integers(0, cin, 36), 4] = 1
+    else:
+        x[5, 9, 50], x[12, 30, 70] = np.nan, np.inf
+    x = x.reshape(-1, cin)
+    raw, wv = weight_bytes(np.ascontiguousarray(w.reshape(cout, -1), np.float32), F16)
+    y = gpu_conv(sess, f"conv:sample:{case}", x, wd, ht, raw, F16, k, k, cin, cout)
+    with np.errstate(invalid="ignore"):
+        ref, top = conv64(x, wd, ht, wv, k), conv64(np.abs(x), wd, ht, np.abs(wv), k)
+    finite = np.isfinite(ref)
+    assert np.array_equal(np.isfinite(y), finite)
+    err = np.abs(y - ref)[finite] / np.maximum(top[finite], 1e-37)
+    print(f"{case}: worst {err.max():.2e} of an output's own terms", flush=True)
+    assert err.max() <= THREE_PRODUCTS
+    assert np.all(y[top == 0] == 0)
 
 
 def test_vae_shape_band_and_translation(sess):
