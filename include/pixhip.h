@@ -495,7 +495,11 @@ int pixhip_conv_weight_get(pixhip_session* session, const char* key, const void*
  * offset kernel / 2, out = in); otherwise out_width = (width + left + right -
  * kernel_x) / stride_x + 1 (and likewise in y), with the reference's checks.
  * Within 1e-4 of the fp32 reference per output row (split products on MFMA,
- * fp32 accumulation): each output within 2^-15 of its own sum |x| |w|.  Tensors are device or pinned host memory (input and
+ * fp32 accumulation): each output within 2^-15 of its own sum |x| |w|.  Images that leave CUs idle are computed in
+ * pieces of the inner sum, in up to 50 MB of the session's memory; a call whose
+ * stream is being captured, or that finds no memory, adds it in one piece (the
+ * fp32 sums are then in another order), and uses nothing of the session's that
+ * a later call could free.  Tensors are device or pinned host memory (input and
  * bias may be pageable), 4-byte aligned.  Images of more than 2^32 - 1 pixels
  * are PIXHIP_ERR_ARGUMENT. */
 int pixhip_conv2d(pixhip_session* session, const pixhip_weight* weight, const float* input, size_t width, size_t height,

@@ -1999,15 +1999,15 @@ int pixhip_conv2d(pixhip_session* s, const pixhip_weight* wc, const float* input
     a.N = (int)w->rows;
     a.Npad = (int)w->conv_npad;
     a.M = (long long)(ow * oh);
-    // The workspace of a split inner range is wanted, not needed: without it
-    // (no memory, or the stream is being captured, when nothing may be
-    // allocated) the call runs whole.
+    // The workspace of a split inner range is wanted, not needed: without the
+    // memory the call runs whole.  So does every call that is being captured,
+    // whatever the session already has: a graph must not hold a workspace that
+    // a later call may free, or use while the graph runs.
     int pieces = pixhip::conv_pieces(a);
-    const size_t part_bytes = (size_t)pieces * out_bytes;
-    if (pieces > 1 && part_bytes > s->partial_bytes) {
+    if (pieces > 1) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s->stream,&capture) != hipSuccess) (void)hipGetLastError();
-        if (capture != hipStreamCaptureStatusNone || grow(s,&s->partial,&s->partial_bytes,part_bytes)) pieces = 1;
+        if (capture != hipStreamCaptureStatusNone || grow(s,&s->partial,&s->partial_bytes,(size_t)pieces * out_bytes)) pieces = 1;
     }
     hipError_t e = pixhip::launch_conv(a,pieces,pieces > 1? static_cast<float*>(s->partial) : nullptr,s->stream);
     if (e == hipErrorInvalidValue) return fail(PIXHIP_ERR_ARGUMENT,"convolution grid too large");

@@ -393,6 +393,50 @@ def test_pinned_host_operands(sess):
     assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("wtype", [F32, F16])
+def test_captured_calls_hold_no_workspace(wtype):
+    """A convolution that eager calls run in pieces, captured into a graph after
+    one of them: the graph keeps nothing of the session's, so that it gives the
+    same bits again while eager calls use the workspace between the replays and
+    larger ones replace it."""
+    rng = np.random.default_rng(17)
+    wd, ht, cin, cout = 24, 20, 256, 64
+    x = rng.standard_normal((wd * ht, cin)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin * 9)) / np.sqrt(cin * 9)).astype(np.float32)
+    raw, wv = weight_bytes(w, wtype)
+    ref = conv2d(oracle(), x, wd, ht, wv, 3, 3)
+    s = new_session()
+    lib, stream, graph, ready = s.lib, ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    try:
+        assert lib.hipStreamCreate(ctypes.byref(stream)) == 0
+        _lib.check(lib.pixhip_session_set_stream(s.handle, stream), "set_stream")
+        eager = gpu_conv(s, "captured", x, wd, ht, raw, wtype, 3, 3, cin, cout)
+        h, xb, yb = s.conv_weight("captured", raw, wtype, 3, 3, cin, cout), s.to_device(x), s.alloc(wd * ht * cout * 4)
+        s.synchronize()
+        assert lib.hipStreamBeginCapture(stream, 1) == 0  # (this thread's calls)
+        rc = s.conv2d(h, xb.ptr, wd, ht, yb.ptr)
+        assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0 and rc == _lib.OK
+        assert lib.hipGraphInstantiate(ctypes.byref(ready), graph, None, None, ctypes.c_size_t(0)) == 0
+        replays = []
+        for side in (24, 32, 40, 44):
+            print(f"replay, then {side} x {side} eager", flush=True)
+            assert lib.hipGraphLaunch(ready, stream) == 0
+            replays.append(yb.download(np.float32, wd * ht * cout).reshape(-1, cout))
+            big = rng.standard_normal((side * side, cin)).astype(np.float32)
+            gpu_conv(s, "captured", big, side, side, raw, wtype, 3, 3, cin, cout)
+            assert np.array_equal(gpu_conv(s, "captured", x, wd, ht, raw, wtype, 3, 3, cin, cout).view(np.uint32), eager.view(np.uint32))
+        assert row_rel_error(replays[0], ref).max() <= TOL and row_rel_error(eager, ref).max() <= TOL
+        for y in replays[1:]:
+            assert np.array_equal(y.view(np.uint32), replays[0].view(np.uint32))
+        assert not np.array_equal(eager, replays[0]), "the eager calls did not run in pieces"
+        s.synchronize()
+        assert lib.hipGraphExecDestroy(ready) == 0 and lib.hipGraphDestroy(graph) == 0
+        _lib.check(lib.pixhip_session_set_stream(s.handle, None), "set_stream")
+        assert lib.hipStreamDestroy(stream) == 0
+    finally:
+        s.close()
+
+
 def test_errors(sess):
     arg, uns = _lib.ERR_ARGUMENT, _lib.ERR_UNSUPPORTED
     raw = np.zeros(4 * 8 * 9 * 2, np.uint8)
