@@ -634,9 +634,9 @@ int matvec(pixhip_session* s, pixhip_weight* w, const float* x, const pixhip::Ou
 // activations are a view of the session's buffers for all rows (which they
 // hold afterwards, as after an unchunked call) and its GEMM reads that view.
 // Taken only when the chunks' GEMMs and the whole one run the same kernel
-// form with no split-K, so every output is the same bits either way.  (Grids
-// small enough for the few-token K-quant form split, or have one super-block,
-// which that form adds the same way.)
+// form with no split-K, so every output is the same bits either way.  (Where
+// the whole call runs a few-token form, so do its chunks: the bits of those do
+// not depend on the rows of a call.)
 size_t pipe_chunk(size_t columns) { return round_up((columns + kPipeChunks - 1) / kPipeChunks,kTileM); }
 
 bool pipeline_ok(const pixhip_weight* w, size_t columns)
@@ -665,6 +665,7 @@ int run_pipelined(pixhip_session* s, pixhip_weight* w, const float* input, size_
         if (!e) PIX_HIP(hipEventCreateWithFlags(&e,hipEventDisableTiming),"hipEventCreate");
     int rc = ensure_gemm_form(s,w);
     if (rc) return rc;
+    const bool few = kind == 1? pixhip::gemm_kq_rows(columns,N,K) : pixhip::gemm_q8_rows(columns,N,K);
     const size_t in_region = round_up(columns * K * sizeof(float),kAlign);
     if ((rc = grow(s,&s->stage,&s->stage_bytes,in_region + columns * N * sizeof(float)))) return rc;
     if ((rc = act_buffers(s,kind,columns,K,nullptr))) return rc;
@@ -687,16 +688,17 @@ int run_pipelined(pixhip_session* s, pixhip_weight* w, const float* input, size_
             const size_t kp = round_up(K,64);
             const pixhip::Act80 a = {s->a80.qs + r0 * kp,s->a80.d + r0,s->a80.mpad};
             PIX_HIP(pixhip::launch_quantize_q8_0(xs + r0 * K,rows,K,kp,a,nullptr,s->stream),"quantize Q8_0");
-            // (the few-token form's bits do not depend on the rows of a call)
-            e = pixhip::gemm_q8_rows(columns,N,K)? pixhip::launch_gemm_rows_q8_0(a,w->q80,rows,N,K,out,s->stream)
-                                                 : pixhip::launch_gemm_q8_0(a,w->q80,rows,N,K,out,part,s->stream);
+            e = few? pixhip::launch_gemm_rows_q8_0(a,w->q80,rows,N,K,out,s->stream)
+                   : pixhip::launch_gemm_q8_0(a,w->q80,rows,N,K,out,part,s->stream);
         } else {
             // tiled planes: rows r0.. (r0 a multiple of 32) start r0*K bytes in, the
             // 16-value sums r0*K/16 elements in; the scales r0 columns in
             const pixhip::Act8K a = {s->a8k.qs + r0 * K,s->a8k.d + r0,s->a8k.bs + r0 * (K / 16),s->a8k.mpad};
             PIX_HIP(pixhip::launch_quantize_q8_K(xs + r0 * K,rows,K,a,nullptr,s->stream),"quantize Q8_K");
-            e = w->type == PIX_Q5_K? pixhip::launch_gemm_q5_K(a,w->q5,rows,N,K,out,part,s->stream)
-                                   : pixhip::launch_gemm_q6_K(a,w->q6,rows,N,K,out,part,s->stream);
+            if (few && w->type == PIX_Q5_K) e = pixhip::launch_gemm_rows_q5_K(a,w->q5,rows,N,K,out,s->stream);
+            else if (few) e = pixhip::launch_gemm_rows_q6_K(a,w->q6,rows,N,K,out,s->stream);
+            else if (w->type == PIX_Q5_K) e = pixhip::launch_gemm_q5_K(a,w->q5,rows,N,K,out,part,s->stream);
+            else e = pixhip::launch_gemm_q6_K(a,w->q6,rows,N,K,out,part,s->stream);
         }
         PIX_HIP(e,"GEMM launch");
         PIX_HIP(hipEventRecord(out_ready,s->stream),"hipEventRecord");
