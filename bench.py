@@ -676,7 +676,7 @@ def bench_surface(sess, synth, _lib):
     return out
 
 
-# VAE convolutions (implicit GEMM on split-bf16 MFMA): (width, height, cin, cout, kernel)
+# VAE convolutions (implicit GEMM on split 16-bit MFMA): (width, height, cin, cout, kernel)
 CONV_CASES = [(256, 256, 512, 512, 3), (1024, 1024, 128, 128, 3), (128, 128, 16, 512, 3)]
 
 

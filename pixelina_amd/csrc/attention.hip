@@ -976,7 +976,7 @@ __global__ __launch_bounds__(kAThreads, 1) void attn_wide_kernel(AttnArgs a)
 // Bound by HBM latency and the launches: a step of 32 heads over 8 kv heads and
 // 2501 keys of 128 (20.5 MB) took 64 us through the tiled kernel (a 256-query
 // tile for 4 queries, after both split passes), 11.2 us
-// here (8.3 + 3.6 for the merge under the tracer).
+// here (7.5 + 3.6 for the merge under the tracer).
 constexpr int kFewWaves = 4, kFewBatch = 16;       // waves per workgroup, keys per wave and step
 constexpr int kFewStep = kFewWaves * kFewBatch;    // keys per workgroup and step
 constexpr int kFewMax = 32;                        // queries per kv head

@@ -535,8 +535,8 @@ __device__ __forceinline__ ConvProbe conv_probe(const ConvArgs& a, uint16_t* lds
 // (64-byte rows, piece c of row r at c ^ ((r >> 2) & 3), no registers), and
 // the image loads run two stages ahead in two register sets, so a stage's
 // stores to LDS wait on loads issued a whole stage earlier.  LDS: one A stage
-// (hi, lo: 20 KB) + two B slots (hi, lo: 16 KB each) = 52 KB, three
-// workgroups per CU.
+// (hi, lo: 20 KB) + two B slots (16 KB for hi and lo; the second 8 KB where the
+// weight is one plane) = 44 or 52 KB, three workgroups per CU.
 //
 // FORM is how the products are formed:
 //   kConvSplit  three bf16 products of split weights and image;
@@ -876,9 +876,11 @@ static bool image_form(const ConvArgs& a)
 // each; pieces cost about 8 us more and a pass that moves (pieces + 1) fp32
 // images at about 4 TB/s.  The estimate's least is taken.  Measured, us, whole /
 // the pieces taken (F16 weights, 3x3): 40^2 pixels 512 -> 512 (52 tiles) 117.8 /
-// 43, 64^2 (128 tiles) 118 / 66, 200 x 100 128 -> 3 (157 tiles) 36.5 / 24.5,
-// 90^2 384 -> 384 (192 tiles) 92 / 74, 128^2 512 -> 256 (256 tiles) 120 / 112;
-// 1x1 at 30^2 (16 stages) gains nothing and stays whole.
+// 45, 64^2 (128 tiles) 118 / 70, 200 x 100 128 -> 3 (157 tiles) 36.5 / 27,
+// 90^2 384 -> 384 (192 tiles) 92 / 80, 128^2 512 -> 256 (256 tiles) 120 / 117;
+// 1x1 at 30^2 (16 stages) gains nothing and stays whole.  The prices are F16
+// weights' for all: BF16 weights take as many products, F32 weights a quarter
+// longer a stage, so that theirs stay whole a little longer than they should.
 int conv_pieces(const ConvArgs& a)
 {
     const long long tiles = (a.M + 127) / 128 * (a.Npad / kCN), cus = device_cus();

@@ -7,8 +7,10 @@ layer shapes, and at the full 256 x 256 x 512 -> 512 shape a sampled band of
 rows plus translation equivariance (an image shifted by one pixel gives the
 shifted output, bit for bit, away from the border).
 
-The kernel multiplies split-bf16 operands on MFMA with fp32 accumulation, so
-outputs are held to TOL = 1e-4 of each output row's largest magnitude."""
+The kernel multiplies operands split into bf16 or fp16 halves on MFMA with fp32
+accumulation, so outputs are held to TOL = 1e-4 of each output row's largest
+magnitude; those of F16 weights also to what three bf16 products leave of each
+output's own terms."""
 import ctypes
 import os
 
@@ -106,8 +108,8 @@ def test_half_weights_over_the_range(sess, scale, geom):
     """F16 weights multiply the image split in fp16 under a power-of-two scale
     per tile: image values over fp32's range, pixels of very different
     magnitude next to each other (those tiles run the bf16 products), zeros.
-    Held to the bf16 split's own bound per output: 3 * 2^-17 of the largest
-    |x| * sum |w|, the worst case of one output's terms adding up."""
+    Held to 3 * 2^-17 of the largest sum |x| |w| over the outputs of the pixel
+    (channels of different magnitudes, and each output's own sum, are below)."""
     rng = np.random.default_rng(7)
     wd, ht, cin, cout, k = 37, 21, 64, 72, 3
     x = rng.standard_normal((wd * ht, cin)).astype(np.float32)
